@@ -411,3 +411,48 @@ def test_engine_kquant_chunked_prefill_matches_oracle(gpu, orc, monkeypatch, qua
         assert rel_l2(eng.copy_logits(), lg) < 1e-3
         tok = g
     eng.close()
+
+
+@pytest.mark.parametrize("m,n,T,epi", [
+    # K split over 8 waves (T <= 32): 2, 4 and 8 row tiles; 10 half column blocks leave
+    # a ragged last step, 384 columns waves without one
+    (300, 640, 1, 0), (33000, 384, 20, 0), (16480, 256, 32, 1), (544, 384, 31, 5),
+    # over 4 (T <= 64): 2, 4, 8 and 10 row tiles
+    (300, 640, 33, 0), (9000, 384, 64, 0), (24592, 384, 64, 0), (40000, 256, 50, 5),
+    # over 2, and none: 4, 8, 10 and 12 row tiles, ragged last row and token blocks
+    (300, 640, 65, 1), (4112, 128, 129, 0), (9000, 384, 200, 5), (33000, 256, 700, 0), (16480, 256, 300, 2),
+    (20000, 256, 400, 5), (16480, 256, 520, 0)])
+def test_gemm_prefill_work_splits(gpu, orc, m, n, T, epi):
+    """Every work split of the block-FP8 prefill GEMM (row tiles per workgroup, waves
+    along tokens and along K) at the edges of its range, with each epilogue, against the
+    oracle on the first and last tokens and those at 32-token boundaries.  Tolerance:
+    activations keep 16 significant bits (at most 2^-15 = 3e-5 off per product) and fp32
+    sums of at most 640 terms add less than 1e-6; SwiGLU multiplies two such results."""
+    r = synth.rng(1100 + m + n + T)
+    toks = sorted({0, T // 2, T - 1} | {t for t in (31, 32, 63, 64, 127, 128, 255, 256) if t < T})
+    X = r.standard_normal((T, n)).astype(np.float32)
+    Xs = np.ascontiguousarray(X[toks])
+    if epi == 5:
+        I = m // 2 // 8 * 8
+        Wg, Wu = synth.fp8_weight_wide(r, I, n), synth.fp8_weight_wide(r, I, n)
+        sg, su = synth.fp8_scales(r, I, n), synth.fp8_scales(r, I, n)
+        g = orc.gemm_fp8(Wg, sg, Xs).astype(np.float64)
+        with np.errstate(over="ignore"):
+            want = g / (1.0 + np.exp(-g)) * orc.gemm_fp8(Wu, su, Xs).astype(np.float64)
+        got = ops.linear_prefill(ops.Fp8GateUp(Wg, sg, Wu, su), X, epilogue=5)
+    else:
+        W, s = synth.fp8_weight_wide(r, m, n), synth.fp8_scales(r, m, n)
+        lin = ops.Fp8Linear(W, s)
+        y = orc.gemm_fp8(W, s, Xs).astype(np.float64)
+        if epi == 2:  # rows 32b .. 32b+15 gate, 32b+16 .. 32b+31 up
+            y2 = y.reshape(len(toks), -1, 2, 16)
+            with np.errstate(over="ignore"):
+                want = (y2[:, :, 0] / (1.0 + np.exp(-y2[:, :, 0])) * y2[:, :, 1]).reshape(len(toks), -1)
+            got = ops.linear_prefill(lin, X, epilogue=2)
+        else:
+            Y0 = r.standard_normal((T, m)).astype(np.float32) if epi == 1 else None
+            want = y + (Y0[toks] if epi == 1 else 0.0)
+            got = ops.linear_prefill(lin, X, epilogue=epi, Y0=Y0)
+    assert np.isfinite(got).all()
+    for k, t in enumerate(toks):
+        assert rel_l2(got[t], want[k]) <= (2 if epi in (2, 5) else 1) * 3.2e-5, (t, rel_l2(got[t], want[k]))
