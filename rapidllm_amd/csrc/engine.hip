@@ -232,6 +232,10 @@ class Engine {
     const void* pf_f16_src_ = nullptr;
     size_t pf_attn_ws_bytes_ = 0;
     int* pf_pos_ = nullptr;
+    // inputs as fp16 + e4m3 parts (prefill_x.hip), for chunks of at least kPfXMin tokens
+    static constexpr int kPfXMin = 64;
+    void *pf_fx_ = nullptr, *pf_fxh_ = nullptr;
+    bool pf_use_x_ = false;  // the current chunk's linears take them
     uint16_t *pf_whi_ = nullptr, *pf_wlo_ = nullptr;  // a K-quant linear as BF16 hi + lo tiles
     float* pf_u_ = nullptr;                          // up rows of separate K-quant gate / up
     std::unique_ptr<DevAlloc> pf_mem_;
@@ -283,9 +287,29 @@ class Engine {
         return e;
     }
 
-    // One prefill linear over T tokens of fragments: Y (=, +=, SwiGLU) W . x.
-    void pf_linear(const Lin& L, const void* frag, float* Y, int ldy, int m_valid, int T, int epi) {
-        if (L.kind == RL_Q_FP8_E4M3_B128) {
+    // Input of the prefill linears: bf16 hi + mid fragments and / or fp16 + e4m3 parts
+    // (x.h null: not written).
+    struct PfIn {
+        const void* frag = nullptr;
+        ActX x;
+    };
+    // Linears that take the fp16 + e4m3 input: block-FP8, and K-quant in the fp16 form.
+    static bool x_kind(const Lin& L) { return L.kind == RL_Q_FP8_E4M3_B128 || (is_kq(L) && kq_f16()); }
+
+    // One prefill linear over T tokens: Y (=, +=, SwiGLU) W . x; out: the next linear's
+    // input (kEpiSwiGLUHX).
+    void pf_linear(const Lin& L, const PfIn& in, float* Y, int ldy, int m_valid, int T, int epi,
+                   const ActX* out = nullptr) {
+        const void* frag = in.frag;
+        if (in.x.h && x_kind(L)) {
+            if (L.kind == RL_Q_FP8_E4M3_B128) {
+                gemm_x(0, L.w, L.ts, in.x, Y, L.m, L.n, T, epi, ldy, m_valid, st_, out);
+            } else {
+                kq_to_f16(L.kind == RL_Q_Q4_K ? 4 : 6, L.w, pf_whi_, pf_ts_, L.m, L.n, st_);
+                gemm_x(3, reinterpret_cast<const uint8_t*>(pf_whi_), pf_ts_, in.x, Y, L.m, L.n, T, epi, ldy, m_valid, st_,
+                       out);
+            }
+        } else if (L.kind == RL_Q_FP8_E4M3_B128) {
             gemm_prefill_any(0, L.w, nullptr, L.ts, frag, Y, L.m, L.n, T, epi, ldy, m_valid, st_);
         } else if (L.kind == RL_Q_BF16) {
             gemm_prefill_any(1, L.w, nullptr, nullptr, frag, Y, L.m, L.n, T, epi, ldy, m_valid, st_);
@@ -306,6 +330,38 @@ class Engine {
                              nullptr, frag, Y, L.m, L.n, T, epi, ldy, m_valid, st_);
         }
     }
+    // RMSNorm of the residual rows as the input of `parts`, in the form(s) they take.
+    PfIn pf_norm(const float* gamma, std::initializer_list<const std::vector<Lin>*> lists,
+                 std::initializer_list<const Lin*> one, int T) {
+        bool need_x = false, need_f = false;
+        auto see = [&](const Lin& L) { (pf_use_x_ && x_kind(L) ? need_x : need_f) = true; };
+        for (const auto* v : lists)
+            for (const Lin& L : *v) see(L);
+        for (const Lin* L : one) see(*L);
+        PfIn in;
+        if (need_f) in.frag = pf_frag_;
+        if (need_x) {
+            in.x = act_x_at(pf_fx_, c_.hidden, T);
+            rmsnorm_x(pf_x_, gamma, in.x, need_f ? pf_frag_ : nullptr, c_.hidden, T, c_.rms_eps, st_);
+        } else {
+            rmsnorm_pack(pf_x_, c_.hidden, gamma, nullptr, pf_frag_, c_.hidden, T, c_.rms_eps, st_);
+        }
+        pf_f16_src_ = nullptr;
+        return in;
+    }
+    // fp32 rows [T][n] as the input of L (memory: pf_fx_ / pf_frag_, or the MLP's pair)
+    PfIn pf_pack(const float* rows, int n, const Lin& L, void* frag, void* fx, int T) {
+        PfIn in;
+        if (pf_use_x_ && x_kind(L) && n % 8 == 0) {
+            in.x = act_x_at(fx, n, T);
+            pack_x(rows, in.x, n, T, st_);
+        } else {
+            in.frag = frag;
+            pack_act(rows, frag, n, T, st_);
+        }
+        pf_f16_src_ = nullptr;
+        return in;
+    }
     // K-quant prefill linears as fp16 tiles (RL_PF_KQ16=0: the BF16 hi + lo tiles)
     static bool kq_f16() {
         static const bool on = [] {
@@ -314,8 +370,8 @@ class Engine {
         }();
         return on;
     }
-    void pf_parts(const std::vector<Lin>& parts, const std::vector<int>& offs, float* Y, int ldy, int T) {
-        for (size_t k = 0; k < parts.size(); ++k) pf_linear(parts[k], pf_frag_, Y + offs[k], ldy, parts[k].m, T, kEpiStore);
+    void pf_parts(const std::vector<Lin>& parts, const std::vector<int>& offs, const PfIn& in, float* Y, int ldy, int T) {
+        for (size_t k = 0; k < parts.size(); ++k) pf_linear(parts[k], in, Y + offs[k], ldy, parts[k].m, T, kEpiStore);
     }
 
     void ensure_pf_buffers(int C) {
@@ -341,6 +397,8 @@ class Engine {
         }
         pf_frag_ = pf_mem_->get(act_frag_bytes(wf, C));
         pf_frag_h_ = pf_mem_->get(act_frag_bytes(I, C));
+        pf_fx_ = pf_mem_->get(act_x_bytes(wf, C));
+        pf_fxh_ = pf_mem_->get(act_x_bytes(I, C));
         pf_attn_ws_bytes_ = attn_prefill_workspace_bytes(std::max(c_.n_q, 1), C);
         pf_attn_ws_ = pf_mem_->get(pf_attn_ws_bytes_);
         pf_pos_ = pf_mem_->get_n<int>(64);
@@ -377,54 +435,74 @@ class Engine {
             const int T = std::min(C, N - c0);
             upload_ints(pf_pos_, &c0, 1);
             embed_rows(embed_, embed_kind_, tok_all_ + c0, pf_x_, H, c_.vocab, T, st_);
+            pf_use_x_ = T >= kPfXMin && rmsnorm_x_supported(H);
             for (int i = 0; i < c_.n_layers; ++i) {
                 Layer& Ly = L_[i];
-                rmsnorm_pack(pf_x_, H, Ly.attn_norm, nullptr, pf_frag_, H, T, eps, st_);
-                pf_f16_src_ = nullptr;
+                const std::vector<Lin>& mix = Ly.kind == RL_LAYER_DELTA ? Ly.in_parts : Ly.qkv_parts;
+                const PfIn in = pf_norm(Ly.attn_norm, {&mix}, {}, T);
                 if (Ly.kind == RL_LAYER_DELTA) {
-                    pf_parts(Ly.in_parts, Ly.in_offs, pf_y_, Ly.in_width, T);
+                    pf_parts(Ly.in_parts, Ly.in_offs, in, pf_y_, Ly.in_width, T);
                     float* ring = slot_conv(Ly.dslot);
                     gdn_prefill(pf_y_, Ly.in_width, Ly.off_a, Ly.off_b, Ly.A_log, Ly.dt_bias, Ly.conv_w,
                                 ring + slot * conv_slot_, ring + (slot ^ 1) * conv_slot_, pf_xc_, pf_gates_,
                                 slot_S(Ly.dslot), pf_o_, T, nk, nv, c_.k_dim, dv, c_.conv_k, c_.v_tiled, st_,
                                 pf_gdn_ck_);
-                    gnorm_pack(pf_o_, pf_y_ + Ly.off_z, Ly.in_width, Ly.gnorm, Ly.gnorm_n, nullptr, pf_frag_, zdim, T,
-                               1e-6f, st_);
+                    const float* z = pf_y_ + Ly.off_z;
+                    PfIn oin;
+                    if (pf_use_x_ && x_kind(Ly.out_proj) && Ly.gnorm_n == 128 && zdim >= 256 && zdim % 128 == 0 &&
+                        Ly.off_z % 4 == 0 && Ly.in_width % 4 == 0) {
+                        oin.x = act_x_at(pf_fx_, zdim, T);
+                        gnorm_x(pf_o_, z, Ly.in_width, Ly.gnorm, oin.x, nullptr, zdim, T, 1e-6f, st_);
+                    } else {
+                        oin.frag = pf_frag_;
+                        gnorm_pack(pf_o_, z, Ly.in_width, Ly.gnorm, Ly.gnorm_n, nullptr, pf_frag_, zdim, T, 1e-6f, st_);
+                    }
                     pf_f16_src_ = nullptr;
-                    pf_linear(Ly.out_proj, pf_frag_, pf_x_, H, H, T, kEpiAdd);
+                    pf_linear(Ly.out_proj, oin, pf_x_, H, H, T, kEpiAdd);
                 } else {
-                    pf_parts(Ly.qkv_parts, Ly.qkv_offs, pf_y_, Ly.qkv_width, T);
+                    pf_parts(Ly.qkv_parts, Ly.qkv_offs, in, pf_y_, Ly.qkv_width, T);
                     attn_prefill_layer(pf_y_, Ly.qkv_width, Ly.q_norm, Ly.k_norm, slot_kc(Ly.aslot), slot_vt(Ly.aslot),
                                        ctx_, pf_pos_, T, nq, nkv, hd, c_.rotary_dim, c_.rope_theta, eps, pf_attn_ws_,
                                        pf_attn_ws_bytes_, pf_o_, st_);
-                    pack_act(pf_o_, pf_frag_, nq * hd, T, st_);
+                    const PfIn oin = pf_pack(pf_o_, nq * hd, Ly.o_proj, pf_frag_, pf_fx_, T);
+                    pf_linear(Ly.o_proj, oin, pf_x_, H, H, T, kEpiAdd);
+                }
+                const bool separate = Ly.gate_up.kind < 0 && !Ly.gate_cat;
+                const Lin& gu = Ly.gate_up.kind >= 0 ? Ly.gate_up : Ly.gate;
+                const bool half_tiles = Ly.gate_up.kind >= 0 ? Ly.gate_up.guh : Ly.gate_cat;
+                PfIn min;
+                if (separate) {
+                    min = pf_norm(Ly.ffn_norm, {}, {&Ly.gate, &Ly.up}, T);
+                } else if (half_tiles) {
+                    min = pf_norm(Ly.ffn_norm, {}, {&gu}, T);
+                } else {  // interleaved whole tiles: the fragments' kernels only
+                    min.frag = pf_frag_;
+                    rmsnorm_pack(pf_x_, H, Ly.ffn_norm, nullptr, pf_frag_, H, T, eps, st_);
                     pf_f16_src_ = nullptr;
-                    pf_linear(Ly.o_proj, pf_frag_, pf_x_, H, H, T, kEpiAdd);
                 }
-                rmsnorm_pack(pf_x_, H, Ly.ffn_norm, nullptr, pf_frag_, H, T, eps, st_);
-                pf_f16_src_ = nullptr;
-                // half-tile gate / up pairs write the down projection's input
-                // fragments directly when I fills whole 128-column blocks
-                const bool h_frag = I % 128 == 0;
-                float* hy = h_frag ? static_cast<float*>(pf_frag_h_) : pf_h_;
-                const int he = h_frag ? kEpiSwiGLUHFrag : kEpiSwiGLUH;
-                bool packed = false;
-                if (Ly.gate_up.kind >= 0 && Ly.gate_up.guh) {
-                    pf_linear(Ly.gate_up, pf_frag_, hy, I, I, T, he);
-                    packed = h_frag;
-                } else if (Ly.gate_up.kind >= 0) {
-                    pf_linear(Ly.gate_up, pf_frag_, pf_h_, I, I, T, Ly.gate_up.swiglu_epi());
-                } else if (Ly.gate_cat) {
-                    pf_linear(Ly.gate, pf_frag_, hy, I, I, T, he);
-                    packed = h_frag;
+                // half-tile gate / up pairs write the down projection's input directly, in
+                // the form both take, when I fills whole 128-column blocks
+                const bool gu_x = min.x.h != nullptr;
+                PfIn din;
+                if (half_tiles && I % 128 == 0 && gu_x && x_kind(Ly.down)) {
+                    din.x = act_x_at(pf_fxh_, I, T);
+                    pf_linear(gu, min, nullptr, I, I, T, kEpiSwiGLUHX, &din.x);
+                    pf_f16_src_ = nullptr;
+                } else if (half_tiles && I % 128 == 0 && !gu_x && !(pf_use_x_ && x_kind(Ly.down))) {
+                    din.frag = pf_frag_h_;
+                    pf_linear(gu, min, static_cast<float*>(pf_frag_h_), I, I, T, kEpiSwiGLUHFrag);
+                    pf_f16_src_ = nullptr;
                 } else {
-                    pf_linear(Ly.gate, pf_frag_, pf_h_, I, I, T, kEpiStore);
-                    pf_linear(Ly.up, pf_frag_, pf_u_, I, I, T, kEpiStore);
-                    swiglu(pf_h_, I, pf_u_, I, pf_h_, I, T, st_);
+                    if (separate) {
+                        pf_linear(Ly.gate, min, pf_h_, I, I, T, kEpiStore);
+                        pf_linear(Ly.up, min, pf_u_, I, I, T, kEpiStore);
+                        swiglu(pf_h_, I, pf_u_, I, pf_h_, I, T, st_);
+                    } else {
+                        pf_linear(gu, min, pf_h_, I, I, T, half_tiles ? kEpiSwiGLUH : Ly.gate_up.swiglu_epi());
+                    }
+                    din = pf_pack(pf_h_, I, Ly.down, pf_frag_h_, pf_fxh_, T);
                 }
-                if (!packed) pack_act(pf_h_, pf_frag_h_, I, T, st_);
-                pf_f16_src_ = nullptr;
-                pf_linear(Ly.down, pf_frag_h_, pf_x_, H, H, T, kEpiAdd);
+                pf_linear(Ly.down, din, pf_x_, H, H, T, kEpiAdd);
             }
             slot ^= 1;
             RL_HIP(hipStreamSynchronize(st_));  // the pinned position stage is reused by the next chunk

@@ -14,7 +14,9 @@ enum GemmEpilogue {
     kEpiSwiGLUH = 5,
     // prefill only: SwiGLU over half tiles written straight as the next GEMM's bf16
     // hi + mid input fragments (Y is the fragment buffer; outputs a multiple of 128)
-    kEpiSwiGLUHFrag = 6
+    kEpiSwiGLUHFrag = 6,
+    // gemm_x only: SwiGLU over half tiles written as the next gemm_x's input
+    kEpiSwiGLUHX = 7
 };
 
 // RMSNorm folded across a residual GEMM and the next linear (y = rmsnorm(x) * (1+g)
@@ -80,6 +82,27 @@ void act_frag_to_f16(const void* frag, void* frag16, float* xscale, int n, int T
 void gemm_fp8_prefill(const uint8_t* W, const float* ts, const void* frag, float* Y, int m, int n, int T, int epi,
                       int ldy, int m_valid, hipStream_t s);
 int device_cus();  // CUs of the current device
+
+// prefill_x.hip: prefill linears over activations as fp16 + e4m3 parts (the layout is
+// described there); act_x_bytes(n, T) bytes of memory hold one input.
+struct ActX {
+    i32x4* h = nullptr;
+    i32x4* l = nullptr;
+    float* s = nullptr;
+};
+size_t act_x_bytes(int n, int T);
+ActX act_x_at(void* mem, int n, int T);
+bool rmsnorm_x_supported(int n);
+// rows x [T][n] (frag, when given: the bf16 hi + mid fragments as well)
+void rmsnorm_x(const float* x, const float* gamma, const ActX& out, void* frag, int n, int T, float eps, hipStream_t s);
+// per 128-wide head, as gnorm_pack with gamma_n = 128
+void gnorm_x(const float* o, const float* z, int ld_z, const float* gamma, const ActX& out, void* frag, int n, int T,
+             float eps, hipStream_t s);
+void pack_x(const float* X, const ActX& out, int n, int T, hipStream_t s);
+// wk 0: block-FP8 tiles; 3: fp16 tiles (kq_to_f16).  epi: store, add, SwiGLU over half
+// tiles, or kEpiSwiGLUHX (m a multiple of 256, the outputs go to *out)
+void gemm_x(int wk, const uint8_t* W, const float* ts, const ActX& x, float* Y, int m, int n, int T, int epi, int ldy,
+            int m_valid, hipStream_t s, const ActX* out = nullptr);
 void pack_act(const float* X, void* frag, int n, int T, hipStream_t s);
 void pack_fp8_rows(const uint8_t* w, const float* scale, uint8_t* dst, float* tscale, int m, int n, int rt_stride,
                    int rt_offset, hipStream_t s);

@@ -456,3 +456,38 @@ def test_gemm_prefill_work_splits(gpu, orc, m, n, T, epi):
     assert np.isfinite(got).all()
     for k, t in enumerate(toks):
         assert rel_l2(got[t], want[k]) <= (2 if epi in (2, 5) else 1) * 3.2e-5, (t, rel_l2(got[t], want[k]))
+
+
+@pytest.mark.parametrize("quant,hidden,inter,T", [
+    # one 128-row and one ragged token block; the MLP's SwiGLU straight into the down
+    # projection's fp16 + e4m3 input (768 rows: three 256-row blocks)
+    ("fp8", 256, 384, 64), ("fp8", 384, 640, 129), ("fp8", 256, 1024, 260),
+    # an intermediate that leaves a partial column block: fp32 SwiGLU rows, then packed
+    ("fp8", 256, 328, 191), ("fp8", 128, 136, 65),
+    ("q4_k", 256, 512, 64), ("q6_k", 512, 768, 257), ("q4_k", 256, 1280, 127),
+    # one token short of the split inputs: the bf16 hi + mid kernels
+    ("fp8", 256, 384, 63), ("q4_k", 256, 512, 63)])
+def test_engine_prefill_split_inputs(gpu, orc, quant, hidden, inter, T):
+    """Prompt chunks of T tokens at the edges of the fp16 + e4m3 prefill linears (64
+    tokens and up; row blocks of 128 to 256, token blocks of 128 and 256, every producer
+    of their inputs) against the oracle model.  Tolerance: block-FP8 inputs are 2^-16
+    off at most, 3e-5 after a few layers; the K-quant weights as fp16 2^-12, 1e-3."""
+    from oracle.oracle import OracleModel
+    from rapidllm_amd import model as M
+    from rapidllm_amd.engine import Engine
+    spec = M.ModelSpec(vocab=512, hidden=hidden, n_layers=4, intermediate=inter, n_k_heads=2, n_v_heads=4, n_q=4,
+                       n_kv=2, layer_kinds=[0, 1, 0, 0], has_mtp=False)
+    lq = {"fp8": M.Q_FP8, "q4_k": M.Q_Q4_K, "q6_k": M.Q_Q6_K}[quant]
+    kw = {"w_scale": (1e-3, 1e-2)} if quant == "fp8" else {"head_quant": M.Q_Q6_K}
+    W = M.random_weights(spec, seed=21 + T, linear_quant=lq, **kw)
+    eng = Engine(spec, W, ctx=512)
+    orc_m = OracleModel(spec, W, ctx=512)
+    prompt = [int(t) for t in np.random.default_rng(T).integers(0, spec.vocab, T + 4)]  # the last 4: a decode step
+    eng.prefill(prompt)
+    orc_m.reset()
+    for t in prompt:
+        g, lg, hd = orc_m.decode(t)
+    bar = 1e-4 if quant == "fp8" else 1e-3
+    assert rel_l2(eng.copy_logits(), lg) < bar, rel_l2(eng.copy_logits(), lg)
+    assert rel_l2(eng.copy_last_hidden(), hd) < bar
+    eng.close()
