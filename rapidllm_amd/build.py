@@ -28,6 +28,11 @@ FLAGS = [
     "-Wno-unused-result",
 ]
 
+# attn_prefill.hip: MFMA results in vector registers also where a kernel may use all 512 (the
+# default puts them in accumulation registers, and every vector instruction on the
+# prefill attention's output would move it over and back).
+FILE_FLAGS = {"attn_prefill.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+
 
 def sources():
     return sorted(glob.glob(os.path.join(CSRC, "*.hip")) + glob.glob(os.path.join(CSRC, "*.cpp")))
@@ -35,9 +40,10 @@ def sources():
 
 def _compile(src: str) -> str:
     obj = os.path.join(OUT_DIR, "obj", os.path.basename(src) + ".o")
-    cmd = [HIPCC, *FLAGS, "-c", src, "-o", obj]
+    flags = FLAGS + FILE_FLAGS.get(os.path.basename(src), [])
+    cmd = [HIPCC, *flags, "-c", src, "-o", obj]
     if src.endswith(".cpp"):
-        cmd = [HIPCC, *FLAGS, "-x", "hip", "-c", src, "-o", obj]
+        cmd = [HIPCC, *flags, "-x", "hip", "-c", src, "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src}:\n{r.stderr}")

@@ -23,80 +23,17 @@
 //
 // Cache layouts: K and V fp16 [n_kv][ctx * hd] in MFMA fragment order (k_off / v_off
 // below); ctx % 256 == 0.
-#include "internal.h"
+#include "attn.h"
 
 using namespace rl;
 
 namespace {
 
-constexpr int kHD = 256;
-constexpr int kChunk = 256;
-constexpr int kMaxPairs = 32;  // G * T query rows per kv head (<= 2 tiles of 16)
 #ifndef ATTN_UNROLL
 #define ATTN_UNROLL 2
 #endif
 
 typedef _Float16 half4 __attribute__((ext_vector_type(4)));
-
-__device__ inline float sigmoid_f(float x) { return 1.f / (1.f + expf(-x)); }
-
-struct AttnArgs {
-    const float* Y;  // fused q(+gate)/k/v projection output, [T][ld_y]
-    int ld_y;
-    const float* q_norm;
-    const float* k_norm;
-    uint16_t* kc;  // [nkv][ctx][hd]
-    uint16_t* vt;  // [nkv][hd][ctx]
-    int ctx;
-    const int* pos;  // device: position of token 0
-    int T, nq, nkv, G, rot;
-    int t_off, T_out;  // outputs: token t goes to column t_off + t of T_out
-    float theta, eps;
-    i32x4* qf;     // [nkv][8 s][4 g][2*PT ct][16 col] x 16 B
-    float* part_o; // [nkv][chunks][kMaxPairs][hd]
-    float* part_m; // [nkv][chunks][kMaxPairs]
-    float* part_l;
-    int max_chunks;
-    float* out;     // optional [T][nq*hd]
-    i32x4* frag;    // optional o_proj fragments (n = nq*hd)
-    // batch decode: nb sequences ("slots") in one launch set.  Slot b's token t is
-    // row b*T + t of Y and output column t_off + b*T + t; its cache, position and
-    // workspace (qf, partials) sit kv_bstride elements, pos_stride ints and ws_slot
-    // bytes after slot b-1's.
-    int nb;
-    size_t kv_bstride;
-    int pos_stride;
-    size_t ws_slot;
-};
-
-// Arguments of slot b (uniform per workgroup: the offsets stay in scalar registers).
-__device__ inline void to_slot(AttnArgs& p, int b) {
-    p.kc += b * p.kv_bstride;
-    p.vt += b * p.kv_bstride;
-    p.pos += b * p.pos_stride;
-    p.Y += static_cast<size_t>(b) * p.T * p.ld_y;
-    p.qf = reinterpret_cast<i32x4*>(reinterpret_cast<char*>(p.qf) + b * p.ws_slot);
-    p.part_o = reinterpret_cast<float*>(reinterpret_cast<char*>(p.part_o) + b * p.ws_slot);
-    p.part_m = reinterpret_cast<float*>(reinterpret_cast<char*>(p.part_m) + b * p.ws_slot);
-    p.part_l = reinterpret_cast<float*>(reinterpret_cast<char*>(p.part_l) + b * p.ws_slot);
-    p.t_off += b * p.T;
-}
-
-__host__ __device__ inline int pair_tiles(int G, int T) { return (G * T + 15) / 16; }
-
-// Cache layouts (per kv head, ctx * 256 fp16), in MFMA fragment order so that every
-// wave load is one contiguous 1 KiB run (lane l reads 16 B at 16 l), and the 4 waves
-// of a chunk workgroup read adjacent runs at every step (one 16 KiB stretch):
-//   K: [pos/256][d/32][(pos/16)%16][(d/8)%4][pos%16][d%8] -- A operand of S^T = K . Q^T
-//   V: [pos/32][d/16][(pos/8)%4][d%16][pos%8]              -- A operand of O^T = V^T . P^T
-__host__ __device__ inline size_t k_off(int pos, int d) {
-    return ((((static_cast<size_t>(pos >> 8) * 8 + (d >> 5)) * 16 + ((pos >> 4) & 15)) * 4 + ((d >> 3) & 3)) * 16 +
-            (pos & 15)) * 8 +
-           (d & 7);
-}
-__host__ __device__ inline size_t v_off(int pos, int d) {
-    return (((static_cast<size_t>(pos >> 5) * 16 + (d >> 4)) * 4 + ((pos >> 3) & 3)) * 16 + (d & 15)) * 8 + (pos & 7);
-}
 
 // grid (nq + 2*nkv, T, slots), 64 threads.  Heads [0,nq): q; [nq, nq+nkv): k; then v.
 __global__ __launch_bounds__(64) void qk_prep_kernel(AttnArgs p) {
@@ -159,12 +96,6 @@ __global__ __launch_bounds__(64) void qk_prep_kernel(AttnArgs p) {
         qf[((base + 2 * pt + 1) * 16 + col) * 8 + e] = lo;
     }
 }
-
-union H8 {
-    f16x8 v;
-    i32x4 i;
-    _Float16 h[8];
-};
 
 template <int PT>
 __global__ __launch_bounds__(256) void attn_part_kernel(AttnArgs p) {
@@ -412,19 +343,16 @@ __global__ __launch_bounds__(64 * kCombG) void attn_comb_kernel(AttnArgs p) {
     }
 }
 
-// ------------------------------------------------------------------ prefill
-// Prompt prefill over T tokens at positions p0 .. p0+T-1 (the reference's prefill
-// attention, cuda_engine.cu:18338-18590, causal GQA over the cache): one
-// workgroup per (block of 16 tokens, kv head, group of up to 3 of its G heads)
-// streams the kv head's cache for those heads x 16 tokens, keeping a running max / sum / O per
-// query row across 256-position chunks (online softmax) -- no partials to combine.
-// Per chunk: S^T = K . Q^T (wave w: positions 64w .. 64w+63, hi and lo parts of q
-// in one accumulator), the chunk max and the rescale of O through LDS, P staged
-// as fp16 by position, O^T += V^T . P^T (wave w: dims 64w .. 64w+63).
+// ---- prefill over short contexts (attn_prefill_is_short): one workgroup per (16 tokens,
+// kv head, up to 3 of its G heads) streams the kv head's cache in chunks of 256 positions, 4
+// waves of 64 positions each, P through LDS.  Two launches and many small workgroups: 64
+// tokens over 64 positions 19.8 us against 31.3 us for the kernels of attn_prefill.hip, 450
+// over 450 43.9 against 51.6, 64 over 764 34.7 against 38.4; over longer contexts those win
+// (700 over 700 75 against 72, 64 over 1264 48.8 against 44.0, 450 over 1250 78 against 66).
 
 // grid (nq + 2*nkv, T), 64 threads: norm + RoPE + cache write as qk_prep_kernel; q
 // goes to qp[kv][tb][s][g][q][hi/lo][16 col] (16 B each; col = token % 16).
-__global__ __launch_bounds__(64) void qk_prep_pf_kernel(AttnArgs p, i32x4* __restrict__ qp) {
+__global__ __launch_bounds__(64) void qk_prep_short_kernel(AttnArgs p, i32x4* __restrict__ qp) {
     __shared__ float vec[kHD];
     const int head = blockIdx.x, t = blockIdx.y, lane = threadIdx.x;
     const int pos = *p.pos + t;
@@ -486,7 +414,7 @@ __global__ __launch_bounds__(64) void qk_prep_pf_kernel(AttnArgs p, i32x4* __res
 // output accumulators stay in registers).
 // Output o[t][h*hd + d] = softmax(q.K/sqrt(hd)) V * sigmoid(gate).
 template <int QT>
-__global__ __launch_bounds__(256) void attn_prefill_kernel(AttnArgs p, const i32x4* __restrict__ qp,
+__global__ __launch_bounds__(256) void attn_prefill_short_kernel(AttnArgs p, const i32x4* __restrict__ qp,
                                                             float* __restrict__ out) {
     const int tb = blockIdx.x, kv = blockIdx.y, q0 = blockIdx.z * QT;
     const int G = p.G;
@@ -718,50 +646,19 @@ void attn_decode_layer(const float* Y, int ld_y, const float* q_norm, const floa
 }
 
 
-size_t attn_prefill_workspace_bytes(int nq, int T) {
-    return static_cast<size_t>(nq) * ((T + 15) / 16) * 16 * kHD * 2 * 2 + 256;
-}
-
-void attn_prefill_layer(const float* Y, int ld_y, const float* q_norm, const float* k_norm, uint16_t* kc,
-                        uint16_t* vt, int ctx, const int* pos_dev, int T, int nq, int nkv, int hd, int rot,
-                        float theta, float eps, void* ws, size_t ws_bytes, float* out, hipStream_t s) {
-    RL_REQUIRE(hd == kHD, RL_ERR_UNSUPPORTED, "attn prefill: head_dim must be 256");
-    RL_REQUIRE(nkv > 0 && nq % nkv == 0, RL_ERR_RANGE, "attn prefill: n_q must be a multiple of n_kv");
-    const int G = nq / nkv;
-    RL_REQUIRE(G >= 1 && G <= 8, RL_ERR_UNSUPPORTED, "attn prefill: n_q/n_kv must be in 1..8");
-    RL_REQUIRE(T >= 1 && T <= 65535 * 16, RL_ERR_RANGE, "attn prefill: bad token count");
-    RL_REQUIRE(ctx > 0 && ctx % kChunk == 0, RL_ERR_RANGE, "attn prefill: cache capacity must be a multiple of 256");
-    RL_REQUIRE(rot >= 2 && rot % 2 == 0 && rot <= hd, RL_ERR_RANGE, "attn prefill: bad rotary dim");
-    RL_REQUIRE(Y && kc && vt && pos_dev && ws && out, RL_ERR_RANGE, "attn prefill: null pointer");
-    RL_REQUIRE(ws_bytes >= attn_prefill_workspace_bytes(nq, T), RL_ERR_RANGE, "attn prefill: workspace too small");
-    AttnArgs p{};
-    p.Y = Y;
-    p.ld_y = ld_y;
-    p.q_norm = q_norm;
-    p.k_norm = k_norm;
-    p.kc = kc;
-    p.vt = vt;
-    p.ctx = ctx;
-    p.pos = pos_dev;
-    p.T = T;
-    p.nq = nq;
-    p.nkv = nkv;
-    p.G = G;
-    p.rot = rot;
-    p.theta = theta;
-    p.eps = eps;
-    i32x4* qp = static_cast<i32x4*>(ws);
-    hipLaunchKernelGGL(qk_prep_pf_kernel, dim3(nq + 2 * nkv, T), dim3(64), 0, s, p, qp);
-    check_launch("qk_prep_pf_kernel");
+void attn_prefill_short(const AttnArgs& p, i32x4* qp, float* out, hipStream_t s) {
+    hipLaunchKernelGGL(qk_prep_short_kernel, dim3(p.nq + 2 * p.nkv, p.T), dim3(64), 0, s, p, qp);
+    check_launch("qk_prep_short_kernel");
     // query tiles per workgroup: 3, 2 or 1 (a divisor of G; four spill registers)
+    const int G = p.G;
     const int QT = G % 3 == 0 ? 3 : G % 2 == 0 ? 2 : 1;
-    const dim3 grid((T + 15) / 16, nkv, G / QT);
+    const dim3 grid((p.T + 15) / 16, p.nkv, G / QT);
     switch (QT) {
-    case 3: hipLaunchKernelGGL(attn_prefill_kernel<3>, grid, dim3(256), 0, s, p, qp, out); break;
-    case 2: hipLaunchKernelGGL(attn_prefill_kernel<2>, grid, dim3(256), 0, s, p, qp, out); break;
-    default: hipLaunchKernelGGL(attn_prefill_kernel<1>, grid, dim3(256), 0, s, p, qp, out); break;
+    case 3: hipLaunchKernelGGL(attn_prefill_short_kernel<3>, grid, dim3(256), 0, s, p, qp, out); break;
+    case 2: hipLaunchKernelGGL(attn_prefill_short_kernel<2>, grid, dim3(256), 0, s, p, qp, out); break;
+    default: hipLaunchKernelGGL(attn_prefill_short_kernel<1>, grid, dim3(256), 0, s, p, qp, out); break;
     }
-    check_launch("attn_prefill_kernel");
+    check_launch("attn_prefill_short_kernel");
 }
 
 }  // namespace rl
@@ -777,18 +674,6 @@ int rl_hip_attn_decode_layer(const float* Y, int ld_y, const float* q_norm, cons
     return guard([&] {
         rl::attn_decode_layer(Y, ld_y, q_norm, k_norm, k_cache, vt_cache, ctx, pos_dev, T, n_q, n_kv, head_dim,
                               rotary_dim, theta, eps, workspace, workspace_bytes, out, frag, S(stream));
-    });
-}
-
-size_t rl_hip_attn_prefill_workspace_bytes(int n_q, int T) { return rl::attn_prefill_workspace_bytes(n_q, T); }
-
-int rl_hip_attn_prefill_layer(const float* Y, int ld_y, const float* q_norm, const float* k_norm, uint16_t* k_cache,
-                              uint16_t* vt_cache, int ctx, const int* pos_dev, int T, int n_q, int n_kv, int head_dim,
-                              int rotary_dim, float theta, float eps, void* workspace, size_t workspace_bytes,
-                              float* out, void* stream) {
-    return guard([&] {
-        rl::attn_prefill_layer(Y, ld_y, q_norm, k_norm, k_cache, vt_cache, ctx, pos_dev, T, n_q, n_kv, head_dim,
-                               rotary_dim, theta, eps, workspace, workspace_bytes, out, S(stream));
     });
 }
 

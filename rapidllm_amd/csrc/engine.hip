@@ -463,7 +463,7 @@ class Engine {
                     pf_parts(Ly.qkv_parts, Ly.qkv_offs, in, pf_y_, Ly.qkv_width, T);
                     attn_prefill_layer(pf_y_, Ly.qkv_width, Ly.q_norm, Ly.k_norm, slot_kc(Ly.aslot), slot_vt(Ly.aslot),
                                        ctx_, pf_pos_, T, nq, nkv, hd, c_.rotary_dim, c_.rope_theta, eps, pf_attn_ws_,
-                                       pf_attn_ws_bytes_, pf_o_, st_);
+                                       pf_attn_ws_bytes_, pf_o_, st_, c0 + T);
                     const PfIn oin = pf_pack(pf_o_, nq * hd, Ly.o_proj, pf_frag_, pf_fx_, T);
                     pf_linear(Ly.o_proj, oin, pf_x_, H, H, T, kEpiAdd);
                 }

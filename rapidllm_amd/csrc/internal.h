@@ -254,7 +254,8 @@ void attn_decode_layer(const float* Y, int ld_y, const float* q_norm, const floa
 size_t attn_prefill_workspace_bytes(int nq, int T);
 void attn_prefill_layer(const float* Y, int ld_y, const float* q_norm, const float* k_norm, uint16_t* kc,
                         uint16_t* vt, int ctx, const int* pos_dev, int T, int nq, int nkv, int hd, int rot,
-                        float theta, float eps, void* ws, size_t ws_bytes, float* out, hipStream_t s);
+                        float theta, float eps, void* ws, size_t ws_bytes, float* out, hipStream_t s,
+                        int max_keys = 0);  // *pos_dev + T at most, if known
 
 // sample.hip
 size_t argmax_workspace_bytes(int rows, int V);

@@ -491,3 +491,53 @@ def test_engine_prefill_split_inputs(gpu, orc, quant, hidden, inter, T):
     assert rel_l2(eng.copy_logits(), lg) < bar, rel_l2(eng.copy_logits(), lg)
     assert rel_l2(eng.copy_last_hidden(), hd) < bar
     eng.close()
+
+
+@pytest.mark.parametrize("T,pos,nq,nkv", [
+    (1, 5000, 24, 4), (17, 3000, 24, 4), (33, 0, 6, 1), (64, 4031, 24, 4), (100, 2500, 12, 2), (65, 1800, 8, 8),
+    (31, 900, 9, 3),      # a kv head count that does not divide the XCDs
+    (1380, 700, 24, 4),   # one full round of workgroups and a split remainder
+    (1366, 0, 24, 4)])    # ... whose ranges start at the first position
+def test_attn_prefill_split_positions(gpu, T, pos, nq, nkv):
+    """Prefill attention where workgroups are split over ranges of positions and merged
+    (few tokens over a long context, and the remainder after full rounds), on the first
+    and last tokens and those around 32-token blocks, against 64-bit attention over the
+    fp16 cache.  Tolerance: probabilities rounded to fp16 (2^-12 each) and a cache entry
+    that rounds the other way (2^-11), below 1e-3 of the output."""
+    r = synth.rng(70 + pos + T + nq)
+    hd, rot, theta = 256, 64, 1e7
+    ctx = ((pos + T + 255) // 256) * 256 + 256
+    Y = r.standard_normal((T, 2 * nq * hd + 2 * nkv * hd)).astype(np.float32)
+    qn = (r.standard_normal(hd) * 0.1).astype(np.float32)
+    kn = (r.standard_normal(hd) * 0.1).astype(np.float32)
+    K = r.standard_normal((pos, nkv, hd)).astype(np.float16).astype(np.float32)
+    V = r.standard_normal((pos, nkv, hd)).astype(np.float16).astype(np.float32)
+    cache = ops.AttnCache(nkv, ctx, hd)
+    if pos:
+        cache.fill(K, V)
+    out = ops.attn_prefill_layer(Y, cache, pos, qn, kn, nq, nkv)
+
+    def norm_rope(x, g):  # [T][heads][256]
+        x = x.astype(np.float64)
+        x = x / np.sqrt((x * x).mean(-1, keepdims=True) + 1e-6) * (1.0 + g.astype(np.float64))
+        freq = (np.float32(1) / np.power(np.float32(theta), np.arange(rot // 2, dtype=np.float32) / (rot // 2)))
+        ang = (np.arange(pos, pos + T, dtype=np.float32)[:, None] * freq.astype(np.float32)).astype(np.float64)[:, None]
+        a, b = x[..., :rot // 2].copy(), x[..., rot // 2:rot].copy()
+        x[..., :rot // 2] = a * np.cos(ang) - b * np.sin(ang)
+        x[..., rot // 2:rot] = a * np.sin(ang) + b * np.cos(ang)
+        return x
+
+    qg = Y[:, :2 * nq * hd].reshape(T, nq, 2, hd)
+    kv = Y[:, 2 * nq * hd:].reshape(T, 2, nkv, hd)
+    q = norm_rope(qg[:, :, 0], qn)
+    Ka = np.concatenate([K, norm_rope(kv[:, 0], kn).astype(np.float16)]).astype(np.float64)
+    Va = np.concatenate([V, kv[:, 1].astype(np.float16)]).astype(np.float64)
+    for t in sorted({0, T // 2, T - 1} | {x for x in (15, 16, 31, 32, 1279, 1280, 1343, 1344) if x < T}):
+        n = pos + t + 1
+        want = np.empty((nq, hd))
+        for h in range(nq):
+            s = Ka[:n, h * nkv // nq] @ q[t, h] / 16.0
+            w = np.exp(s - s.max())
+            want[h] = (w / w.sum()) @ Va[:n, h * nkv // nq]
+        want /= 1.0 + np.exp(-qg[t, :, 1].astype(np.float64))
+        assert rel_l2(out[t], want.reshape(-1)) < 1e-3, (t, rel_l2(out[t], want.reshape(-1)))
