@@ -872,7 +872,12 @@ constexpr int kCk = 64;          // tokens per chunk
 constexpr int kCkStride = kDK + 4;  // LDS row stride of q / k (floats)
 constexpr int kCkA = kCk + 4;       // LDS row stride of A
 // one (v-head, chunk) block of the workspace: U~ [64][128] | W~ [64][128] |
-// gamma Q [64][128] | K~^T [128][64] | M [64][64]
+// gamma Q [64][128] | K~^T [128][64] | M [64][64], each in the order the scan's lanes take
+// it, so that a wave's load is one contiguous 1 KiB run: 16 x 16 tiles (row-major) of 64
+// float4, the A operands' unit lane (g, r) = row r, columns 4g .. 4g + 3 of the tile, and
+// U~'s = rows 4g .. 4g + 3, column r (a C operand).  As plain rows each load took 64 bytes
+// of 16 rows, and the scan waited for its operands (2011 tokens, 48 heads: scan 230 -> 184
+// us, prep 125 -> 140 us for the pass of W~ through LDS, all of the prefill 382 -> 338 us).
 constexpr size_t kCkFloats = 4 * static_cast<size_t>(kCk) * kDK + static_cast<size_t>(kCk) * kCk;
 
 __device__ inline f32x4 mfma_f32_4(float a, float b, f32x4 c) {
@@ -956,10 +961,10 @@ __global__ __launch_bounds__(256, 2) void gdn_pf_chunk_prep_kernel(GdnPfArgs p, 
     __syncthreads();
     // gamma Q rows (q is not needed after the products below)
     for (int u = tid; u < kCk * kDK / 4; u += 256) {
-        const int t = u / (kDK / 4), d = (u % (kDK / 4)) * 4;
+        const int t = 16 * (u >> 9) + (u & 15), d = 16 * ((u >> 6) & 7) + 4 * ((u >> 4) & 3);
         const float gm = expf(static_cast<float>(la_s[t]));
         const float4 qv = *reinterpret_cast<const float4*>(&q_s[t][d]);
-        *reinterpret_cast<float4*>(qg + t * kDK + d) = make_float4(gm * qv.x, gm * qv.y, gm * qv.z, gm * qv.w);
+        reinterpret_cast<float4*>(qg)[u] = make_float4(gm * qv.x, gm * qv.y, gm * qv.z, gm * qv.w);
     }
     // K K^T and Q K^T by 16 x 16 tiles on MFMA; M to memory, A kept until q is free
     f32x4 at[4];
@@ -990,7 +995,7 @@ __global__ __launch_bounds__(256, 2) void gdn_pf_chunk_prep_kernel(GdnPfArgs p, 
             const int t = 16 * tb + 4 * g + e;
             const float G = i <= t ? expf(static_cast<float>(la_s[t] - la_s[i])) : 0.f;
             at[jb][e] = i < t ? beta_s[t] * G * kk[e] : 0.f;
-            m[t * kCk + i] = G * qk[e];
+            m[((tb * 4 + ib) * 64 + (r >> 2) * 16 + 4 * g + e) * 4 + (r & 3)] = G * qk[e];
         }
     }
     __syncthreads();
@@ -1015,19 +1020,28 @@ __global__ __launch_bounds__(256, 2) void gdn_pf_chunk_prep_kernel(GdnPfArgs p, 
         for (int i = 0; i < t; ++i) s4[i & 3] = fmaf(-a_s[t][i], x[i], s4[i & 3]);
         x[t] = (s4[0] + s4[1]) + (s4[2] + s4[3]);
     }
-    {
-        float* dst = col < kDK ? ut + col : wt + (col - kDK);
+    __syncthreads();  // A is not needed any more: its buffer takes W~ on the way to tile order
+    if (col < kDK) {
 #pragma unroll
-        for (int t = 0; t < kCk; ++t) dst[t * kDK] = x[t];
+        for (int t = 0; t < kCk; t += 4)
+            reinterpret_cast<float4*>(ut)[((t >> 4) * 8 + (col >> 4)) * 64 + ((t >> 2) & 3) * 16 + (col & 15)] =
+                make_float4(x[t], x[t + 1], x[t + 2], x[t + 3]);
+    } else {
+#pragma unroll
+        for (int t = 0; t < kCk; ++t) q_s[t][col - kDK] = x[t];
     }
+    __syncthreads();
+    for (int u = tid; u < kCk * kDK / 4; u += 256)
+        reinterpret_cast<float4*>(wt)[u] = *reinterpret_cast<const float4*>(
+            &q_s[16 * (u >> 9) + (u & 15)][16 * ((u >> 6) & 7) + 4 * ((u >> 4) & 3)]);
     // K~ transposed
     for (int u = tid; u < kDK * kCk / 4; u += 256) {
-        const int d = u / (kCk / 4), t = (u % (kCk / 4)) * 4;
+        const int d = 16 * (u >> 8) + (u & 15), t = 16 * ((u >> 6) & 3) + 4 * ((u >> 4) & 3);
         float v[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e)
             v[e] = expf(static_cast<float>(la_s[n - 1] - la_s[t + e])) * k_s[t + e][d];
-        *reinterpret_cast<float4*>(ktT + d * kCk + t) = make_float4(v[0], v[1], v[2], v[3]);
+        reinterpret_cast<float4*>(ktT)[u] = make_float4(v[0], v[1], v[2], v[3]);
     }
     if (tid == 0) gc[static_cast<size_t>(h) * nch + c] = expf(static_cast<float>(la_s[n - 1]));
 }
@@ -1046,7 +1060,7 @@ __device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_b
 template <int NCT>
 struct CkOpsA {
     float4 wa[kDK / 16], qa[kDK / 16];
-    float uu[NCT][4];
+    float4 uu[NCT];
 };
 struct CkOpsB {
     float4 ma[kCk / 16], ka[2][kCk / 16];
@@ -1069,31 +1083,27 @@ __global__ __launch_bounds__(256, 3 - NCT) void gdn_pf_chunk_scan_kernel(GdnPfAr
     const int h = blockIdx.x % p.nv, j0 = (blockIdx.x / p.nv) * NC;
     __shared__ __align__(16) float st_s[NC][kDK + 4];  // state block transposed: [column][key row]
     __shared__ __align__(16) float ut_s[NC][kCk + 4];  // U transposed: [column][token]
-    const int row = 16 * w + r;
     auto blk = [&](int c) { return ws + (static_cast<size_t>(h) * nch + c) * kCkFloats; };
     auto load_a = [&](int c, CkOpsA<NCT>& o) {
-        const float* ut = blk(c);
-        const float* wt = ut + kCk * kDK;
-        const float* qg = wt + kCk * kDK;
+        const float4* ut = reinterpret_cast<const float4*>(blk(c)) + 8 * w * 64 + lane;
+        const float4* wt = ut + kCk * kDK / 4;
+        const float4* qg = wt + kCk * kDK / 4;
 #pragma unroll
         for (int s = 0; s < kDK / 16; ++s) {
-            o.wa[s] = *reinterpret_cast<const float4*>(wt + row * kDK + 16 * s + 4 * g);
-            o.qa[s] = *reinterpret_cast<const float4*>(qg + row * kDK + 16 * s + 4 * g);
+            o.wa[s] = wt[s * 64];
+            o.qa[s] = qg[s * 64];
         }
 #pragma unroll
-        for (int ct = 0; ct < NCT; ++ct)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) o.uu[ct][e] = ut[(16 * w + 4 * g + e) * kDK + j0 + 16 * ct + r];
+        for (int ct = 0; ct < NCT; ++ct) o.uu[ct] = ut[(j0 / 16 + ct) * 64];
     };
     auto load_b = [&](int c, CkOpsB& o) {
-        const float* ktT = blk(c) + 3 * kCk * kDK;
-        const float* m = ktT + kDK * kCk;
+        const float4* ktT = reinterpret_cast<const float4*>(blk(c) + 3 * kCk * kDK) + lane;
+        const float4* m = ktT + kDK * kCk / 4;
 #pragma unroll
         for (int s = 0; s < kCk / 16; ++s) {
-            o.ma[s] = *reinterpret_cast<const float4*>(m + row * kCk + 16 * s + 4 * g);
+            o.ma[s] = m[(4 * w + s) * 64];
 #pragma unroll
-            for (int tt = 0; tt < 2; ++tt)
-                o.ka[tt][s] = *reinterpret_cast<const float4*>(ktT + (32 * w + 16 * tt + r) * kCk + 16 * s + 4 * g);
+            for (int tt = 0; tt < 2; ++tt) o.ka[tt][s] = ktT[((2 * w + tt) * 4 + s) * 64];
         }
         o.gC = gc[static_cast<size_t>(h) * nch + c];
     };
@@ -1141,9 +1151,8 @@ __global__ __launch_bounds__(256, 3 - NCT) void gdn_pf_chunk_scan_kernel(GdnPfAr
         // U = U~ - W~ S (rows 16w + 4g + e, column 16 ct + r)
 #pragma unroll
         for (int ct = 0; ct < NCT; ++ct) {
-            f32x4 u;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) u[e] = ac.uu[ct][e] - au[ct][e];
+            const f32x4 u = {ac.uu[ct].x - au[ct][0], ac.uu[ct].y - au[ct][1], ac.uu[ct].z - au[ct][2],
+                             ac.uu[ct].w - au[ct][3]};
             *reinterpret_cast<f32x4*>(&ut_s[16 * ct + r][16 * w + 4 * g]) = u;
         }
         load_a(cn, an);
