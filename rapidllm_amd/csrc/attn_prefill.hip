@@ -469,8 +469,9 @@ void attn_prefill_layer(const float* Y, int ld_y, const float* q_norm, const flo
     p.theta = theta;
     p.eps = eps;
     i32x4* qp = static_cast<i32x4*>(ws);
-    // (the position is on the device: the context is at most the cache's capacity)
-    if (attn_prefill_is_short(T, max_keys > 0 ? std::min(max_keys, ctx) : ctx)) {
+    // (the position is on the device: the context is at most the cache's capacity; the
+    // kernel below addresses a head's cache with 32-bit offsets)
+    if (attn_prefill_is_short(T, max_keys > 0 ? std::min(max_keys, ctx) : ctx) || ctx >= 1 << 23) {
         attn_prefill_short(p, qp, out, s);
         return;
     }
