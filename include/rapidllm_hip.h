@@ -276,8 +276,14 @@ int rl_hip_embed_rows(const void* table, int kind, const int* tokens_dev, float*
 /* Prompt prefill of T tokens at positions *pos_dev .. *pos_dev + T - 1: the T tokens'
  * K (after norm + RoPE) and V are written to the caches, then causal attention of
  * every token over positions 0 .. its own, out = [T][n_q*256] fp32 times
- * sigmoid(gate).  One workgroup per (16 tokens, kv head) with an online softmax over
- * 256-position chunks.  Replaces the reference's prefill attention
+ * sigmoid(gate).  Online softmax; up to 768 keys a workgroup takes 16 tokens and chunks
+ * of 256 positions, else four waves of 32 queries share stages of 64 positions, and
+ * workgroups that would not fill the chip are split over positions and merged.  The
+ * position is read on the device, and with it the kernel chosen (a captured call
+ * follows *pos_dev at each replay).  The workspace holds the q fragments and 34 MB for
+ * the split; one of only n_q * ceil(T/16) * 16 KiB + 256 bytes is accepted and nothing is
+ * split.  Outputs are the same from call to call, but the order of a token's sums
+ * depends on T and on the number of keys.  Replaces the reference's prefill attention
  * (cuda_engine.cu:18338-18590; CPU: per token ops::attn_decode, ops.cpp:575-605). */
 size_t rl_hip_attn_prefill_workspace_bytes(int n_q, int T);
 int rl_hip_attn_prefill_layer(const float* Y, int ld_y, const float* q_norm, const float* k_norm, uint16_t* k_cache,

@@ -23,6 +23,8 @@
 //
 // Cache layouts: K and V fp16 [n_kv][ctx * hd] in MFMA fragment order (k_off / v_off
 // below); ctx % 256 == 0.
+#include <algorithm>
+
 #include "attn.h"
 
 using namespace rl;
@@ -414,9 +416,8 @@ __global__ __launch_bounds__(64) void qk_prep_short_kernel(AttnArgs p, i32x4* __
 // output accumulators stay in registers).
 // Output o[t][h*hd + d] = softmax(q.K/sqrt(hd)) V * sigmoid(gate).
 template <int QT>
-__global__ __launch_bounds__(256) void attn_prefill_short_kernel(AttnArgs p, const i32x4* __restrict__ qp,
-                                                            float* __restrict__ out) {
-    const int tb = blockIdx.x, kv = blockIdx.y, q0 = blockIdx.z * QT;
+__device__ void attn_short(const AttnArgs& p, const i32x4* __restrict__ qp, float* __restrict__ out, int tb, int kv,
+                           int q0) {
     const int G = p.G;
     const int ntb = (p.T + 15) / 16;
     const int p0 = *p.pos;
@@ -572,6 +573,29 @@ __global__ __launch_bounds__(256) void attn_prefill_short_kernel(AttnArgs p, con
     }
 }
 
+template <int QT>
+__global__ __launch_bounds__(256) void attn_prefill_short_kernel(AttnArgs p, const i32x4* __restrict__ qp,
+                                                                 float* __restrict__ out) {
+    attn_short<QT>(p, qp, out, blockIdx.x, blockIdx.y, blockIdx.z * QT);
+}
+
+// Last launch of a chunk whose route the device chooses: short contexts whole, else the merge of
+// attn_prefill_kernel's parts (one launch less than both).  One head per workgroup: with three the
+// short side's 403 registers left the merge one workgroup per CU (512 tokens over 4512 keys 141
+// us, now 137) and the short side was slower, too (64 over 64 19.7, now 15.1; 450 over 450 43.3,
+// now 37.5).  The short side inside attn_prefill_kernel's launch instead: 450 over 450 60 us.
+__global__ __launch_bounds__(256) void attn_prefill_finish_kernel(AttnArgs p, const i32x4* __restrict__ qp,
+                                                                  float* __restrict__ out, int items, PfParts pp) {
+    const int b = blockIdx.x;
+    if (attn_prefill_auto_short(*p.pos + p.T)) {
+        const int ntb = (p.T + 15) / 16;
+        if (b < ntb * p.nq) attn_short<1>(p, qp, out, b / p.nq, b % p.nkv, b / p.nkv % p.G);
+    } else if (pp.parts > 1) {
+        const int rows = (items - pp.unsplit) * 4;
+        if (b < rows * p.nkv * 4) merge_parts(p, out, items, pp, b % rows, b / rows % p.nkv, b / rows / p.nkv);
+    }
+}
+
 }  // namespace
 
 namespace rl {
@@ -646,9 +670,13 @@ void attn_decode_layer(const float* Y, int ld_y, const float* q_norm, const floa
 }
 
 
-void attn_prefill_short(const AttnArgs& p, i32x4* qp, float* out, hipStream_t s) {
+void attn_prefill_short_prep(const AttnArgs& p, i32x4* qp, hipStream_t s) {
     hipLaunchKernelGGL(qk_prep_short_kernel, dim3(p.nq + 2 * p.nkv, p.T), dim3(64), 0, s, p, qp);
     check_launch("qk_prep_short_kernel");
+}
+
+void attn_prefill_short(const AttnArgs& p, i32x4* qp, float* out, hipStream_t s) {
+    attn_prefill_short_prep(p, qp, s);
     // query tiles per workgroup: 3, 2 or 1 (a divisor of G; four spill registers)
     const int G = p.G;
     const int QT = G % 3 == 0 ? 3 : G % 2 == 0 ? 2 : 1;
@@ -659,6 +687,13 @@ void attn_prefill_short(const AttnArgs& p, i32x4* qp, float* out, hipStream_t s)
     default: hipLaunchKernelGGL(attn_prefill_short_kernel<1>, grid, dim3(256), 0, s, p, qp, out); break;
     }
     check_launch("attn_prefill_short_kernel");
+}
+
+void attn_prefill_auto_finish(const AttnArgs& p, const i32x4* qp, float* out, int items, const PfParts& pp, hipStream_t s) {
+    const int rows = pp.parts > 1 ? (items - pp.unsplit) * 4 * p.nkv : 0;
+    const dim3 grid(std::max((p.T + 15) / 16 * p.nq, rows * 4));
+    hipLaunchKernelGGL(attn_prefill_finish_kernel, grid, dim3(256), 0, s, p, qp, out, items, pp);
+    check_launch("attn_prefill_finish_kernel");
 }
 
 }  // namespace rl

@@ -18,9 +18,9 @@ constexpr int kPrepLd = kHD + 4;
 // grid (ceil(T / 16) + 1, ceil((nq + 2 nkv) / hpw)), 256 threads: the tokens of one aligned
 // group of 16 positions, hpw of the heads [0, nq) q, [nq, nq + nkv) k, then v.  16 lanes per
 // token (dims 4 l + 64 k) form the norm; the rows go through LDS so that every store is a
-// 16-byte unit of the layouts (q: qp[head][t / 16][d / 16][hi/lo][(d / 8) % 2][t % 16]) and
-// the token's RoPE angles are formed once for the workgroup's heads.  One wave per (head,
-// token), storing 2-byte elements: 44 us for 1500 tokens, 24 + 2 x 4 heads.
+// 16-byte unit of the layouts and the token's RoPE angles are formed once for the
+// workgroup's heads.  One wave per (head, token), storing 2-byte elements: 44 us for 1500
+// tokens, 24 + 2 x 4 heads.
 __global__ __launch_bounds__(256) void qk_prep_pf_kernel(AttnArgs p, i32x4* __restrict__ qp, int hpw) {
     __shared__ float row_s[16][kPrepLd];
     __shared__ float2 ang_s[16][kHD / 2];
@@ -122,10 +122,9 @@ __global__ __launch_bounds__(256) void qk_prep_pf_kernel(AttnArgs p, i32x4* __re
             if (!is_q) {
                 *reinterpret_cast<i32x4*>(p.kc + static_cast<size_t>(head - p.nq) * p.ctx * kHD + k_off(base + j, d)) = hi.v;
             } else {
-                i32x4* o = qp + ((static_cast<size_t>(head) * ntb + (tt >> 4)) * 16 + (d >> 4)) * 64 +
-                           ((d >> 3) & 1) * 16 + (tt & 15);
+                i32x4* o = qp + q_unit(head / p.G, head % p.G, p.G, ntb, tt >> 4) + (d >> 3) * p.G * 32 + (tt & 15);
                 o[0] = hi.v;
-                o[32] = lo.v;
+                o[16] = lo.v;
             }
         }
     }
@@ -133,25 +132,6 @@ __global__ __launch_bounds__(256) void qk_prep_pf_kernel(AttnArgs p, i32x4* __re
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __attribute__((address_space(3))) void lds_void;
-
-// Split positions.  The chip runs one workgroup per CU, so the workgroups past the last
-// full round (all of them, with few tokens) are split into `parts` ranges of positions;
-// each range leaves its output, maximum and sum in the workspace.  The split follows from
-// T and the head counts; a workgroup lowers the number of parts to what its context fills
-// (kMinPartBlocks blocks of 64 positions each).  33 tokens over 8033 positions: 368 -> 62 us.
-struct PfParts {
-    int unsplit;  // workgroups per kv head that take all positions
-    int parts;
-    float* o;     // [kv head][split workgroup][part][4 waves][32 queries][256]
-    float2* ml;   // [...][4 waves][32 queries]: maximum (log2 units), sum
-};
-constexpr int kMinPartBlocks = 2;
-__device__ inline int pf_parts(int parts, int nblk) { return max(1, min(parts, nblk / kMinPartBlocks)); }
-// keys 0 .. L-1 for item i (4 (token block, head) entries) of a kv head
-__device__ inline int pf_keys(int i, int G, int T, int p0) {
-    const int e_last = min(i * 4 + 3, G * ((T + 31) / 32) - 1);
-    return p0 + min(T, 32 * (e_last / G) + 32);
-}
 
 // One workgroup: 4 waves x 32 queries of one kv head (wave: one head, 32 tokens), all
 // reading the same K and V from LDS, where 64 positions of each (32 KiB) are copied
@@ -167,7 +147,9 @@ __device__ inline int pf_keys(int i, int G, int T, int p0) {
 // us and 4.5 ms.  A running maximum that moves only past 2^8 saves the rescaling but
 // rounds the largest probability, otherwise an exact 1 (error 2.06e-4 against 1.93e-4). 
 __global__ __launch_bounds__(256, 1) void attn_prefill_kernel(AttnArgs p, const i32x4* __restrict__ qp,
-                                                              float* __restrict__ out, int items, PfParts pp) {
+                                                              float* __restrict__ out, int items, PfParts pp,
+                                                              int auto_route) {
+    if (auto_route && attn_prefill_auto_short(*p.pos + p.T)) return;  // attn_prefill_finish_kernel has it
     __shared__ i32x4 K0[2048], K1[2048];  // [d/32][pos/16][(d/8)%4][pos%16]
     __shared__ i32x4 V0[2048], V1[2048];  // [pos/32][d/16][(pos/8)%4][d%16]
     // kv head from the XCD (blockIdx % 8), so that its cache is read through one L2 (or
@@ -234,12 +216,11 @@ __global__ __launch_bounds__(256, 1) void attn_prefill_kernel(AttnArgs p, const 
 
     H8 qh[16], ql[16];
     {
-        const i32x4* qq = qp + (static_cast<size_t>(head) * ntb16 + min(2 * tb + (col >> 4), ntb16 - 1)) * 16 * 2 * 32 +
-                          h * 16 + (col & 15);
+        const i32x4* qq = qp + q_unit(kv, e % p.G, p.G, ntb16, min(2 * tb + (col >> 4), ntb16 - 1)) + h * p.G * 32 + (col & 15);
 #pragma unroll
         for (int st = 0; st < 16; ++st) {
-            qh[st].i = qq[st * 64];
-            ql[st].i = qq[st * 64 + 32];
+            qh[st].i = qq[st * p.G * 64];
+            ql[st].i = qq[st * p.G * 64 + 16];
             // q lives in accumulation registers, which the MFMAs read directly: the output
             // is rescaled by vector instructions and has the others
 #pragma unroll
@@ -387,44 +368,9 @@ __global__ __launch_bounds__(256, 1) void attn_prefill_kernel(AttnArgs p, const 
         }
 }
 
-// Adds the parts of the split queries: grid (split items * 4 waves, nkv, 4), 256 threads;
-// wave w of block z adds queries 8z + 2w, 8z + 2w + 1, lane l dims 4l .. 4l+3, parts in order.
+// grid (split items * 4 waves, nkv, 4), 256 threads
 __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs p, float* __restrict__ out, int items, PfParts pp) {
-    const int si = blockIdx.x / 4, wv = blockIdx.x % 4, kv = blockIdx.y;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int item = items - 1 - (pp.unsplit + si);
-    const int e = item * 4 + wv;
-    if (e >= p.G * ((p.T + 31) / 32)) return;
-    const int parts = pf_parts(pp.parts, (pf_keys(item, p.G, p.T, *p.pos) + 63) / 64);
-    if (parts == 1) return;
-    const int head = kv * p.G + e % p.G, tb = e / p.G;
-    const size_t w0 = (static_cast<size_t>(kv) * (items - pp.unsplit) + si) * pp.parts * 4 + wv;
-    for (int q = blockIdx.z * 8 + 2 * wave; q < static_cast<int>(blockIdx.z) * 8 + 2 * wave + 2; ++q) {
-        const int tok = 32 * tb + q;
-        if (tok >= p.T) return;
-        float M = -INFINITY;
-        for (int k = 0; k < parts; ++k) M = fmaxf(M, pp.ml[(w0 + 4 * k) * 32 + q].x);
-        float l = 0.f;
-        float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (int k = 0; k < parts; ++k) {
-            const float2 ml = pp.ml[(w0 + 4 * k) * 32 + q];
-            const float f = __builtin_amdgcn_exp2f(ml.x - M);
-            const float4 o = *reinterpret_cast<const float4*>(pp.o + ((w0 + 4 * k) * 32 + q) * kHD + 4 * lane);
-            l = fmaf(f, ml.y, l);
-            a.x = fmaf(f, o.x, a.x);
-            a.y = fmaf(f, o.y, a.y);
-            a.z = fmaf(f, o.z, a.z);
-            a.w = fmaf(f, o.w, a.w);
-        }
-        const float inv = 1.f / l;
-        const float* gate = p.Y + static_cast<size_t>(tok) * p.ld_y + static_cast<size_t>(head) * 2 * kHD + kHD + 4 * lane;
-        float4 r;
-        r.x = a.x * inv * sigmoid_f(gate[0]);
-        r.y = a.y * inv * sigmoid_f(gate[1]);
-        r.z = a.z * inv * sigmoid_f(gate[2]);
-        r.w = a.w * inv * sigmoid_f(gate[3]);
-        *reinterpret_cast<float4*>(out + static_cast<size_t>(tok) * (p.nq * kHD) + static_cast<size_t>(head) * kHD + 4 * lane) = r;
-    }
+    merge_parts(p, out, items, pp, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
 }  // namespace
@@ -475,12 +421,18 @@ void attn_prefill_layer(const float* Y, int ld_y, const float* q_norm, const flo
         attn_prefill_short(p, qp, out, s);
         return;
     }
+    // a large cache and keys that only the device knows: the kernels choose
+    const bool auto_route = max_keys <= 0 && attn_prefill_auto_short(T);
     // four heads per workgroup share the angles once that still leaves two workgroups per CU
     // (1500 tokens: 31 us); with fewer tokens one head each, for the latency
     const int hpw = ((T + 15) / 16) * (nq + 2 * nkv) >= 8 * device_cus() ? 4 : 1;
-    hipLaunchKernelGGL(qk_prep_pf_kernel, dim3((T + 15) / 16 + 1, (nq + 2 * nkv + hpw - 1) / hpw), dim3(256), 0, s, p, qp,
-                       hpw);
-    check_launch("qk_prep_pf_kernel");
+    if (auto_route) {
+        attn_prefill_short_prep(p, qp, s);
+    } else {
+        hipLaunchKernelGGL(qk_prep_pf_kernel, dim3((T + 15) / 16 + 1, (nq + 2 * nkv + hpw - 1) / hpw), dim3(256), 0, s, p,
+                           qp, hpw);
+        check_launch("qk_prep_pf_kernel");
+    }
     const int items = (G * ((T + 31) / 32) + 3) / 4;  // workgroups per kv head
     // whole rounds of one workgroup per CU take all positions; the rest are split so that
     // they fill a round (with the parts' memory: a workspace of just the q fragments takes
@@ -501,9 +453,12 @@ void attn_prefill_layer(const float* Y, int ld_y, const float* q_norm, const flo
     const int slots = pp.unsplit + (items - pp.unsplit) * pp.parts;  // workgroups per kv head
     const int per = 8 % nkv == 0 ? 8 / nkv : 1;
     const int wgs = 8 % nkv == 0 ? (slots + per - 1) / per * 8 : slots * nkv;
-    hipLaunchKernelGGL(attn_prefill_kernel, dim3(wgs), dim3(256), 0, s, p, qp, out, items, pp);
+    hipLaunchKernelGGL(attn_prefill_kernel, dim3(wgs), dim3(256), 0, s, p, qp, out, items, pp,
+                       static_cast<int>(auto_route));
     check_launch("attn_prefill_kernel");
-    if (pp.parts > 1) {
+    if (auto_route) {
+        attn_prefill_auto_finish(p, qp, out, items, pp, s);
+    } else if (pp.parts > 1) {
         hipLaunchKernelGGL(attn_merge_kernel, dim3((items - pp.unsplit) * 4, nkv, 4), dim3(256), 0, s, p, out, items, pp);
         check_launch("attn_merge_kernel");
     }

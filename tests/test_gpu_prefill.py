@@ -541,3 +541,30 @@ def test_attn_prefill_split_positions(gpu, T, pos, nq, nkv):
             want[h] = (w / w.sum()) @ Va[:n, h * nkv // nq]
         want /= 1.0 + np.exp(-qg[t, :, 1].astype(np.float64))
         assert rel_l2(out[t], want.reshape(-1)) < 1e-3, (t, rel_l2(out[t], want.reshape(-1)))
+
+
+@pytest.mark.parametrize("T,pos,nq,nkv", [
+    (1, 0, 24, 4), (17, 0, 24, 4), (64, 0, 6, 1), (65, 3, 8, 8), (100, 668, 12, 2),   # 768 keys
+    (450, 0, 24, 4), (512, 256, 9, 3), (300, 100, 24, 4), (768, 0, 6, 1),
+    (101, 668, 12, 2), (512, 257, 24, 4), (768, 1, 24, 4), (769, 0, 8, 8)])           # one key more
+def test_attn_prefill_short_context_in_large_cache(gpu, T, pos, nq, nkv):
+    """A chunk over few keys takes the short kernel whatever the cache's capacity: up to 768
+    keys the outputs are the bytes that a cache of just those keys gives.  Beyond, two kernels that each round probabilities to fp16 (2^-12) agree within 1e-3."""
+    r = synth.rng(90 + pos + T + nq)
+    hd = 256
+    Y = r.standard_normal((T, 2 * nq * hd + 2 * nkv * hd)).astype(np.float32)
+    K = r.standard_normal((pos, nkv, hd)).astype(np.float16).astype(np.float32)
+    V = r.standard_normal((pos, nkv, hd)).astype(np.float16).astype(np.float32)
+    qn, kn = (r.standard_normal(hd).astype(np.float32) * np.float32(0.1) for _ in range(2))
+    outs = []
+    for ctx in ((pos + T + 255) // 256 * 256, 8192):
+        cache = ops.AttnCache(nkv, ctx, hd)
+        if pos:
+            cache.fill(K, V)
+        outs.append(ops.attn_prefill_layer(Y, cache, pos, qn, kn, nq, nkv))
+    assert np.isfinite(outs[0]).all()
+    if pos + T <= 768:
+        assert outs[0].tobytes() == outs[1].tobytes()
+    else:
+        for t in range(T):
+            assert rel_l2(outs[1][t], outs[0][t]) < 1e-3, (t, rel_l2(outs[1][t], outs[0][t]))
