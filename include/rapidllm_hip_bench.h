@@ -1,8 +1,9 @@
 /*
  * rapidllm_hip_bench.h -- benchmark, tuning and calibration entry points of the
  * MI355X decode backend.  None has a counterpart in the reference: they serve
- * bench.py and the roofline / profiler measurements, not the engine seam
- * (rapidllm_hip.h), and a RapidLLM integration does not need them.
+ * bench.py, the roofline / profiler measurements and tests of launches that otherwise
+ * only the engine makes, not the engine seam (rapidllm_hip.h), and a RapidLLM
+ * integration does not need them.
  *
  * rl_hip_set_gemm_config changes process-wide state (the GEMM work split every
  * later launch uses); the timing functions launch back-to-back kernels on the given
@@ -99,6 +100,24 @@ int rl_hip_time_gdn(float* const* S_layers, int n_layers, const float* qkv, cons
                     const float* A_log, const float* dt_bias, const float* conv_w, const float* conv_in,
                     float* conv_out, float* o, int T, int nk, int nv, int dk, int dv, int conv_k, int v_tiled,
                     int iters, void* stream, float* avg_ms);
+
+/* ---- the engine's prompt linears alone (tests) --------------------------------
+ * Inputs of T tokens as fp16 + e4m3 parts: kb = ceil(n / 128) column blocks; per input
+ *   h [kb][i 4][g 4][T] 16-byte units, fp16(x / s) of columns 32g + 8i .. + 7
+ *   l [kb][c 2][g 4][T] 16-byte units, e4m3((x / s - h) * 2^7) of columns 32g + 16c .. + 15
+ *   s [kb][T] fp32, a power of two with the block's largest |x| / s in [2^12, 2^13)
+ * one after the other (rl_hip_act_x_bytes bytes).  Elements 2^-14 and more below their
+ * block's largest lose bits of the remainder, from 2^-18 all of them (11 bits are left).
+ * rl_hip_gemm_x: fp16_tiles 0: block-FP8 tiles, 1: the fp16 tiles of rl_hip_kquant_to_f16.
+ * epilogue 0 store, 1 add, 5 SwiGLU over half tiles (m / 2 outputs), 7 the same written as
+ * the next linear's input x_out (m / 2 a multiple of 128).  ldy <= 0: the outputs' number.
+ * rl_hip_gemm_x_split: the launches it makes on `cus` CUs, (64-row blocks per workgroup,
+ * 64-token blocks per workgroup, row blocks) of the first and of the second (0 0 0: none). */
+size_t rl_hip_act_x_bytes(int n, int T);
+int rl_hip_pack_act_x(const float* X, void* x, int n, int T, void* stream);
+int rl_hip_gemm_x(int fp16_tiles, const void* w, const float* tile_scale, const void* x, float* Y, void* x_out, int m, int n,
+                  int T, int epilogue, int ldy, void* stream);
+int rl_hip_gemm_x_split(int fp16_tiles, int epilogue, int m, int T, int cus, int* split);
 
 #ifdef __cplusplus
 }

@@ -452,7 +452,7 @@ class Engine {
                     if (pf_use_x_ && x_kind(Ly.out_proj) && Ly.gnorm_n == 128 && zdim >= 256 && zdim % 128 == 0 &&
                         Ly.off_z % 4 == 0 && Ly.in_width % 4 == 0) {
                         oin.x = act_x_at(pf_fx_, zdim, T);
-                        gnorm_x(pf_o_, z, Ly.in_width, Ly.gnorm, oin.x, nullptr, zdim, T, 1e-6f, st_);
+                        gnorm_x(pf_o_, z, Ly.in_width, Ly.gnorm, oin.x, zdim, T, 1e-6f, st_);
                     } else {
                         oin.frag = pf_frag_;
                         gnorm_pack(pf_o_, z, Ly.in_width, Ly.gnorm, Ly.gnorm_n, nullptr, pf_frag_, zdim, T, 1e-6f, st_);

@@ -96,8 +96,8 @@ bool rmsnorm_x_supported(int n);
 // rows x [T][n] (frag, when given: the bf16 hi + mid fragments as well)
 void rmsnorm_x(const float* x, const float* gamma, const ActX& out, void* frag, int n, int T, float eps, hipStream_t s);
 // per 128-wide head, as gnorm_pack with gamma_n = 128
-void gnorm_x(const float* o, const float* z, int ld_z, const float* gamma, const ActX& out, void* frag, int n, int T,
-             float eps, hipStream_t s);
+void gnorm_x(const float* o, const float* z, int ld_z, const float* gamma, const ActX& out, int n, int T, float eps,
+             hipStream_t s);
 void pack_x(const float* X, const ActX& out, int n, int T, hipStream_t s);
 // wk 0: block-FP8 tiles; 3: fp16 tiles (kq_to_f16).  epi: store, add, SwiGLU over half
 // tiles, or kEpiSwiGLUHX (m a multiple of 256, the outputs go to *out)

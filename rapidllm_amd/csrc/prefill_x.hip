@@ -154,7 +154,7 @@ __global__ __launch_bounds__(256) void rmsnorm_x_kernel(const float* __restrict_
 // Gated RMSNorm per 128-wide head (gnorm_pack128_kernel's arithmetic) as an ActX.
 __global__ __launch_bounds__(256) void gnorm_x_kernel(const float* __restrict__ o, const float* __restrict__ z, int ld_z,
                                                       const float* __restrict__ gamma, ActX out,
-                                                      i32x4* __restrict__ frag, int n, int T, float eps) {
+                                                      int n, int T, float eps) {
     const int t = blockIdx.y, tid = threadIdx.x;
     const int hh = blockIdx.x * 16 + (tid >> 4), u = tid & 15;
     if (hh * 128 >= n) return;  // whole 16-lane groups
@@ -173,7 +173,6 @@ __global__ __launch_bounds__(256) void gnorm_x_kernel(const float* __restrict__ 
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = (gamma ? gamma[8 * u + e] : 1.f) * (ov[e] * inv) * silu_f(zv[e]);
     put_x8(out, c0 >> 3, t, T, v);
-    if (frag) write_frag8(frag, c0 >> 3, t, T, v);
 }
 
 // ------------------------------------------------------------------- the GEMM
@@ -546,64 +545,79 @@ void launch_gemm_x_cfg(GemmX p, int rt_base, int row_blocks, hipStream_t s) {
     check_launch("gemm_x_kernel");
 }
 
-// The work split: 256, 192 or 128 rows (R = 4, 3, 2) x 256 or 128 tokens (TG = 4, 2) per
-// workgroup.  A CU holds one 256-token workgroup, or for block-FP8 two of 128 tokens
-// (their barriers fall at different times: 32768 x 5120, 2048 tokens, 955 against 1037 us);
-// a round of workgroups takes about 2R + 1 units.  A lone 4-wave workgroup on a CU takes
-// 0.65 of that.  When whole rounds leave a small remainder of row blocks, those rows are
-// a launch of their own with another split (34816 rows, 2044 tokens in fp16 tiles: 5
-// rounds of 256 x 256 with the last one a quarter full).
-template <int WK, bool kGuh>
-void launch_gemm_x(const GemmX& p, hipStream_t s) {
-    struct Cfg {
-        int r, tg;
-        void (*launch)(GemmX, int, int, hipStream_t);
-    };
-    static const Cfg cfgs[] = {{4, 4, launch_gemm_x_cfg<WK, kGuh, 4, 4>}, {3, 4, launch_gemm_x_cfg<WK, kGuh, 3, 4>},
-                               {2, 4, launch_gemm_x_cfg<WK, kGuh, 2, 4>}, {4, 2, launch_gemm_x_cfg<WK, kGuh, 4, 2>},
-                               {3, 2, launch_gemm_x_cfg<WK, kGuh, 3, 2>}, {2, 2, launch_gemm_x_cfg<WK, kGuh, 2, 2>}};
-    const int m_tiles = (p.m + kTileRows - 1) / kTileRows, cus = device_cus();
-    const bool x_out = p.epi == kEpiSwiGLUHX;  // whole column blocks of outputs: 256 rows
-    auto blocks = [](const Cfg& c, int tiles) { return (tiles + 4 * c.r - 1) / (4 * c.r); };
-    auto ntb = [&](const Cfg& c) { return (p.T + 64 * c.tg - 1) / (64 * c.tg); };
-    auto slots = [&](const Cfg& c) { return c.tg == 2 && WK == 0 ? 2 * cus : cus; };
-    auto cost = [&](const Cfg& c, long wgs) {
-        const double unit = (2 * c.r + 1) * (c.tg == 4 ? 1.0 : WK == 0 ? 0.95 : 0.65);
+// Row blocks of 64 r rows from a row tile on, in blocks of 64 tg tokens.
+struct XSplit {
+    int r = 0, tg = 0, blocks = 0;
+};
+
+// The work split: 256, 192 or 128 rows (r = 4, 3, 2) x 256 or 128 tokens (tg = 4, 2) per
+// workgroup.  A CU holds one workgroup, and of block-FP8 two of 128 tokens, which is why
+// block-FP8 takes no others (their barriers fall at different times: 32768 x 5120, 2048
+// tokens, 955 us against 1037 with 256 tokens); a round of workgroups takes about 2r + 1
+// units.  A lone 4-wave workgroup on a CU takes 0.65 of that.  When whole rounds leave a
+// small remainder of row blocks, those rows are a launch of their own with another split
+// (34816 rows, 2044 tokens in fp16 tiles: 5 rounds of 256 x 256 with the last one a quarter
+// full).  x_out: outputs in whole column blocks, 256 rows.  The sums of an output do not
+// depend on the split.
+void gemm_x_split(int wk, bool x_out, int m, int T, int cus, XSplit& first, XSplit& rest) {
+    static constexpr XSplit kSplits[] = {{4, 4}, {3, 4}, {2, 4}, {4, 2}, {3, 2}, {2, 2}};
+    const int m_tiles = (m + kTileRows - 1) / kTileRows;
+    auto skip = [&](const XSplit& c) { return (x_out && c.r != 4) || (wk == 0 && c.tg != 2); };
+    auto blocks = [](const XSplit& c, int tiles) { return (tiles + 4 * c.r - 1) / (4 * c.r); };
+    auto ntb = [&](const XSplit& c) { return (T + 64 * c.tg - 1) / (64 * c.tg); };
+    auto slots = [&](const XSplit& c) { return wk == 0 ? 2 * cus : cus; };
+    auto cost = [&](const XSplit& c, long wgs) {
+        const double unit = (2 * c.r + 1) * (c.tg == 4 ? 1.0 : wk == 0 ? 0.95 : 0.65);
         const long full = wgs / slots(c), rem = wgs % slots(c);
-        return unit * (full + (rem == 0 ? 0.0 : c.tg == 2 && WK == 0 && rem <= cus ? 0.65 : 1.0));
+        return unit * (full + (rem == 0 ? 0.0 : wk == 0 && rem <= cus ? 0.65 : 1.0));
     };
-    const Cfg *first = nullptr, *rest = nullptr;
-    int first_blocks = 0;
     double best = 0;
-    for (const Cfg& c : cfgs) {
-        if (x_out && c.r != 4) continue;
+    for (const XSplit& c : kSplits) {
+        if (skip(c)) continue;
         const int nb = blocks(c, m_tiles);
         const long wgs = static_cast<long>(nb) * ntb(c);
         RL_REQUIRE(wgs < (1L << 30), RL_ERR_RANGE, "gemm_x: too many workgroups");
         const double t = cost(c, wgs);
-        if (!first || t < best) {
+        if (!first.blocks || t < best) {
             best = t;
-            first = &c;
-            first_blocks = nb;
-            rest = nullptr;
+            first = {c.r, c.tg, nb};
+            rest = {};
         }
         const int nb1 = static_cast<int>(wgs / slots(c) * slots(c) / ntb(c));
         if (nb1 == 0 || nb1 == nb) continue;
-        for (const Cfg& c2 : cfgs) {
-            if (x_out && c2.r != 4) continue;
+        for (const XSplit& c2 : kSplits) {
+            if (skip(c2)) continue;
             const int nb2 = blocks(c2, m_tiles - nb1 * 4 * c.r);
             // a second launch costs about a third of a unit
             const double t2 = cost(c, static_cast<long>(nb1) * ntb(c)) + cost(c2, static_cast<long>(nb2) * ntb(c2)) + 0.35;
             if (t2 < best) {
                 best = t2;
-                first = &c;
-                first_blocks = nb1;
-                rest = &c2;
+                first = {c.r, c.tg, nb1};
+                rest = {c2.r, c2.tg, nb2};
             }
         }
     }
-    first->launch(p, 0, first_blocks, s);
-    if (rest) rest->launch(p, first_blocks * 4 * first->r, blocks(*rest, m_tiles - first_blocks * 4 * first->r), s);
+}
+
+template <int WK, bool kGuh>
+void launch_gemm_x(const GemmX& p, hipStream_t s) {
+    XSplit first, rest;
+    gemm_x_split(WK, p.epi == kEpiSwiGLUHX, p.m, p.T, device_cus(), first, rest);
+    auto launch = [&](const XSplit& c, int rt_base) {
+        if constexpr (WK == 3) {
+            if (c.tg == 4) {
+                if (c.r == 4) launch_gemm_x_cfg<WK, kGuh, 4, 4>(p, rt_base, c.blocks, s);
+                if (c.r == 3) launch_gemm_x_cfg<WK, kGuh, 3, 4>(p, rt_base, c.blocks, s);
+                if (c.r == 2) launch_gemm_x_cfg<WK, kGuh, 2, 4>(p, rt_base, c.blocks, s);
+                return;
+            }
+        }
+        if (c.r == 4) launch_gemm_x_cfg<WK, kGuh, 4, 2>(p, rt_base, c.blocks, s);
+        if (c.r == 3) launch_gemm_x_cfg<WK, kGuh, 3, 2>(p, rt_base, c.blocks, s);
+        if (c.r == 2) launch_gemm_x_cfg<WK, kGuh, 2, 2>(p, rt_base, c.blocks, s);
+    };
+    launch(first, 0);
+    if (rest.blocks) launch(rest, first.blocks * 4 * first.r);
 }
 
 }  // namespace
@@ -641,13 +655,13 @@ void rmsnorm_x(const float* x, const float* gamma, const ActX& out, void* frag, 
     check_launch("rmsnorm_x_kernel");
 }
 
-void gnorm_x(const float* o, const float* z, int ld_z, const float* gamma, const ActX& out, void* frag, int n, int T,
-             float eps, hipStream_t s) {
+void gnorm_x(const float* o, const float* z, int ld_z, const float* gamma, const ActX& out, int n, int T, float eps,
+             hipStream_t s) {
     RL_REQUIRE(o && z && out.h && n > 0 && n % 128 == 0 && T >= 1 && T <= 65535, RL_ERR_RANGE, "gnorm_x: bad arguments");
     RL_REQUIRE(reinterpret_cast<uintptr_t>(o) % 16 == 0 && reinterpret_cast<uintptr_t>(z) % 16 == 0 && ld_z % 4 == 0,
                RL_ERR_RANGE, "gnorm_x: rows must be 16-byte aligned");
-    hipLaunchKernelGGL(gnorm_x_kernel, dim3((n / 128 + 15) / 16, T), dim3(256), 0, s, o, z, ld_z, gamma, out,
-                       static_cast<i32x4*>(frag), n, T, eps);
+    hipLaunchKernelGGL(gnorm_x_kernel, dim3((n / 128 + 15) / 16, T), dim3(256), 0, s, o, z, ld_z, gamma, out, n, T,
+                       eps);
     check_launch("gnorm_x_kernel");
 }
 
@@ -694,3 +708,39 @@ void gemm_x(int wk, const uint8_t* W, const float* ts, const ActX& x, float* Y, 
 }
 
 }  // namespace rl
+
+extern "C" {
+
+size_t rl_hip_act_x_bytes(int n, int T) { return rl::act_x_bytes(n, T); }
+
+int rl_hip_pack_act_x(const float* X, void* x, int n, int T, void* stream) {
+    return guard([&] {
+        RL_REQUIRE(x && n > 0 && T > 0, RL_ERR_RANGE, "pack_act_x: bad arguments");
+        rl::pack_x(X, rl::act_x_at(x, n, T), n, T, S(stream));
+    });
+}
+
+int rl_hip_gemm_x(int fp16_tiles, const void* w, const float* tile_scale, const void* x, float* Y, void* x_out, int m, int n,
+                  int T, int epilogue, int ldy, void* stream) {
+    return guard([&] {
+        RL_REQUIRE(x && m > 0 && n > 0 && T > 0, RL_ERR_RANGE, "gemm_x: bad arguments");
+        const bool to_x = epilogue == rl::kEpiSwiGLUHX;
+        RL_REQUIRE(!to_x || x_out, RL_ERR_RANGE, "gemm_x: null output");
+        const int mo = to_x || epilogue == rl::kEpiSwiGLUH ? m / 2 : m;
+        const rl::ActX out = to_x ? rl::act_x_at(x_out, mo, T) : rl::ActX{};
+        rl::gemm_x(fp16_tiles ? 3 : 0, static_cast<const uint8_t*>(w), tile_scale, rl::act_x_at(const_cast<void*>(x), n, T),
+                   Y, m, n, T, epilogue, ldy > 0 ? ldy : mo, mo, S(stream), to_x ? &out : nullptr);
+    });
+}
+
+int rl_hip_gemm_x_split(int fp16_tiles, int epilogue, int m, int T, int cus, int* split) {
+    return guard([&] {
+        RL_REQUIRE(m > 0 && T > 0 && cus > 0 && split, RL_ERR_RANGE, "gemm_x_split: bad arguments");
+        XSplit first, rest;
+        gemm_x_split(fp16_tiles ? 3 : 0, epilogue == rl::kEpiSwiGLUHX, m, T, cus, first, rest);
+        const int v[6] = {first.r, first.tg, first.blocks, rest.r, rest.tg, rest.blocks};
+        for (int k = 0; k < 6; ++k) split[k] = v[k];
+    });
+}
+
+}  // extern "C"

@@ -469,8 +469,9 @@ def test_gemm_prefill_work_splits(gpu, orc, m, n, T, epi):
     ("fp8", 256, 384, 63), ("q4_k", 256, 512, 63)])
 def test_engine_prefill_split_inputs(gpu, orc, quant, hidden, inter, T):
     """Prompt chunks of T tokens at the edges of the fp16 + e4m3 prefill linears (64
-    tokens and up; row blocks of 128 to 256, token blocks of 128 and 256, every producer
-    of their inputs) against the oracle model.  Tolerance: block-FP8 inputs are 2^-16
+    tokens and up; every producer of their inputs, in models so small that the linears
+    take 128-token blocks of 128 rows, or of 256 with the SwiGLU output: the other work
+    splits are in test_gpu_gemm_x.py) against the oracle model.  Tolerance: block-FP8 inputs are 2^-16
     off at most, 3e-5 after a few layers; the K-quant weights as fp16 2^-12, 1e-3."""
     from oracle.oracle import OracleModel
     from rapidllm_amd import model as M
