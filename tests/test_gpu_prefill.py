@@ -421,7 +421,9 @@ def test_engine_kquant_chunked_prefill_matches_oracle(gpu, orc, monkeypatch, qua
     (300, 640, 33, 0), (9000, 384, 64, 0), (24592, 384, 64, 0), (40000, 256, 50, 5),
     # over 2, and none: 4, 8, 10 and 12 row tiles, ragged last row and token blocks
     (300, 640, 65, 1), (4112, 128, 129, 0), (9000, 384, 200, 5), (33000, 256, 700, 0), (16480, 256, 300, 2),
-    (20000, 256, 400, 5), (16480, 256, 520, 0)])
+    (20000, 256, 400, 5), (16480, 256, 520, 0),
+    # a second group of eight token blocks, one or two blocks wide
+    (300, 640, 1025, 0), (544, 384, 1160, 5)])
 def test_gemm_prefill_work_splits(gpu, orc, m, n, T, epi):
     """Every work split of the block-FP8 prefill GEMM (row tiles per workgroup, waves
     along tokens and along K) at the edges of its range, with each epilogue, against the
@@ -429,7 +431,7 @@ def test_gemm_prefill_work_splits(gpu, orc, m, n, T, epi):
     activations keep 16 significant bits (at most 2^-15 = 3e-5 off per product) and fp32
     sums of at most 640 terms add less than 1e-6; SwiGLU multiplies two such results."""
     r = synth.rng(1100 + m + n + T)
-    toks = sorted({0, T // 2, T - 1} | {t for t in (31, 32, 63, 64, 127, 128, 255, 256) if t < T})
+    toks = sorted({0, T // 2, T - 1} | {t for t in (31, 32, 63, 64, 127, 128, 255, 256, 1023, 1024, 1151, 1152) if t < T})
     X = r.standard_normal((T, n)).astype(np.float32)
     Xs = np.ascontiguousarray(X[toks])
     if epi == 5:
