@@ -395,12 +395,13 @@ class Engine {
             const size_t ckf = gdn_prefill_chunked() ? gdn_prefill_chunk_floats(C, c_.n_v_heads, c_.k_dim, c_.v_dim) : 0;
             pf_gdn_ck_ = ckf ? pf_mem_->get_n<float>(ckf) : nullptr;
         }
-        pf_frag_ = pf_mem_->get(act_frag_bytes(wf, C));
-        pf_frag_h_ = pf_mem_->get(act_frag_bytes(I, C));
-        pf_fx_ = pf_mem_->get(act_x_bytes(wf, C));
-        pf_fxh_ = pf_mem_->get(act_x_bytes(I, C));
+        // a norm writes both forms of its output where its linears take both; the MLP's input
+        // has one form at a time, and the attention runs between the linears that read
+        // pf_frag_ and the packing of its output
         pf_attn_ws_bytes_ = attn_prefill_workspace_bytes(std::max(c_.n_q, 1), C);
-        pf_attn_ws_ = pf_mem_->get(pf_attn_ws_bytes_);
+        pf_frag_ = pf_attn_ws_ = pf_mem_->get(std::max(act_frag_bytes(wf, C), pf_attn_ws_bytes_));
+        pf_frag_h_ = pf_fxh_ = pf_mem_->get(std::max(act_frag_bytes(I, C), act_x_bytes(I, C)));
+        pf_fx_ = pf_mem_->get(act_x_bytes(wf, C));
         pf_pos_ = pf_mem_->get_n<int>(64);
         const size_t kqe = kq_prefill_elems();
         if (kqe) {

@@ -496,6 +496,32 @@ def test_engine_prefill_split_inputs(gpu, orc, quant, hidden, inter, T):
     eng.close()
 
 
+@pytest.mark.parametrize("quant", ["fp8", "q4_k"])
+def test_engine_prefill_mixed_chunks(gpu, orc, monkeypatch, quant):
+    """One prompt in chunks of both input forms (100 tokens: fp16 + e4m3; 50: bf16 hi + mid),
+    attention and DeltaNet layers, then a second prompt: the forms share buffers.  Bars as in
+    test_engine_prefill_split_inputs."""
+    from oracle.oracle import OracleModel
+    from rapidllm_amd import model as M
+    from rapidllm_amd.engine import Engine
+    monkeypatch.setenv("RL_PREFILL_CHUNK", "100")
+    spec = M.ModelSpec(vocab=512, hidden=256, n_layers=4, intermediate=512, n_k_heads=2, n_v_heads=4, n_q=4, n_kv=2,
+                       layer_kinds=[0, 1, 0, 0], has_mtp=False)
+    kw = {"w_scale": (1e-3, 1e-2)} if quant == "fp8" else {"head_quant": M.Q_Q6_K}
+    W = M.random_weights(spec, seed=77, linear_quant=M.Q_FP8 if quant == "fp8" else M.Q_Q4_K, **kw)
+    eng, orc_m = Engine(spec, W, ctx=512), OracleModel(spec, W, ctx=512)
+    bar = 1e-4 if quant == "fp8" else 1e-3
+    for n, seed in ((154, 1), (254, 2)):
+        prompt = [int(t) for t in np.random.default_rng(seed).integers(0, spec.vocab, n)]
+        eng.reset()
+        eng.prefill(prompt)
+        orc_m.reset()
+        for t in prompt:
+            _, lg, _ = orc_m.decode(t)
+        assert rel_l2(eng.copy_logits(), lg) < bar, (n, rel_l2(eng.copy_logits(), lg))
+    eng.close()
+
+
 @pytest.mark.parametrize("T,pos,nq,nkv", [
     (1, 5000, 24, 4), (17, 3000, 24, 4), (33, 0, 6, 1), (64, 4031, 24, 4), (100, 2500, 12, 2), (65, 1800, 8, 8),
     (31, 900, 9, 3),      # a kv head count that does not divide the XCDs
