@@ -115,6 +115,11 @@ int rl_hip_time_gdn(float* const* S_layers, int n_layers, const float* qkv, cons
  * 64-token blocks per workgroup, row blocks) of the first and of the second (0 0 0: none). */
 size_t rl_hip_act_x_bytes(int n, int T);
 int rl_hip_pack_act_x(const float* X, void* x, int n, int T, void* stream);
+/* RMSNorm of rows (n a multiple of 128, at most 6144), and the DeltaNet layers' gated RMSNorm
+ * per 128-wide head, written as such an input. */
+int rl_hip_rmsnorm_x(const float* rows, const float* gamma, void* x, int n, int T, float eps, void* stream);
+int rl_hip_gated_rmsnorm_x(const float* o, const float* z, int ld_z, const float* gamma, void* x, int n, int T, float eps,
+                           void* stream);
 int rl_hip_gemm_x(int fp16_tiles, const void* w, const float* tile_scale, const void* x, float* Y, void* x_out, int m, int n,
                   int T, int epilogue, int ldy, void* stream);
 int rl_hip_gemm_x_split(int fp16_tiles, int epilogue, int m, int T, int cus, int* split);

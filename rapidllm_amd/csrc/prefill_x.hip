@@ -151,7 +151,7 @@ __global__ __launch_bounds__(256) void rmsnorm_x_kernel(const float* __restrict_
     }
 }
 
-// Gated RMSNorm per 128-wide head (gnorm_pack128_kernel's arithmetic) as an ActX.
+// Gated RMSNorm per 128-wide head (gnorm_pack128_kernel's arithmetic, expf included) as an ActX.
 __global__ __launch_bounds__(256) void gnorm_x_kernel(const float* __restrict__ o, const float* __restrict__ z, int ld_z,
                                                       const float* __restrict__ gamma, ActX out,
                                                       int n, int T, float eps) {
@@ -171,7 +171,8 @@ __global__ __launch_bounds__(256) void gnorm_x_kernel(const float* __restrict__ 
     const float inv = 1.f / sqrtf(static_cast<float>(ss / 128) + eps);
     float v[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = (gamma ? gamma[8 * u + e] : 1.f) * (ov[e] * inv) * silu_f(zv[e]);
+    for (int e = 0; e < 8; ++e)
+        v[e] = (gamma ? gamma[8 * u + e] : 1.f) * (ov[e] * inv) * (zv[e] / (1.f + expf(-zv[e])));
     put_x8(out, c0 >> 3, t, T, v);
 }
 
@@ -717,6 +718,21 @@ int rl_hip_pack_act_x(const float* X, void* x, int n, int T, void* stream) {
     return guard([&] {
         RL_REQUIRE(x && n > 0 && T > 0, RL_ERR_RANGE, "pack_act_x: bad arguments");
         rl::pack_x(X, rl::act_x_at(x, n, T), n, T, S(stream));
+    });
+}
+
+int rl_hip_rmsnorm_x(const float* rows, const float* gamma, void* x, int n, int T, float eps, void* stream) {
+    return guard([&] {
+        RL_REQUIRE(x && n > 0 && T > 0, RL_ERR_RANGE, "rmsnorm_x: bad arguments");
+        rl::rmsnorm_x(rows, gamma, rl::act_x_at(x, n, T), nullptr, n, T, eps, S(stream));
+    });
+}
+
+int rl_hip_gated_rmsnorm_x(const float* o, const float* z, int ld_z, const float* gamma, void* x, int n, int T, float eps,
+                           void* stream) {
+    return guard([&] {
+        RL_REQUIRE(x && n > 0 && T > 0, RL_ERR_RANGE, "gated_rmsnorm_x: bad arguments");
+        rl::gnorm_x(o, z, ld_z, gamma, rl::act_x_at(x, n, T), n, T, eps, S(stream));
     });
 }
 

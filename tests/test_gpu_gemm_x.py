@@ -141,6 +141,33 @@ def test_pack_act_x(gpu, n, T):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,T", [(128, 64), (768, 70), (5120, 65), (6144, 67)])
+def test_norms_to_act_x(gpu, n, T):
+    """The layer norm and the gated norm written as an input are the bytes of the norms that
+    write fp32 rows (rl_hip_rmsnorm_pack, rl_hip_gated_rmsnorm_pack), packed: no less precise.
+    Gates reach far enough down for the exponential's precision to show."""
+    r = synth.rng(n + T)
+    X, g = inputs(r, T, n), (r.standard_normal(n) * 0.1).astype(np.float32)
+    d = [DeviceBuffer.from_numpy(a) for a in (X, g)]
+    y, x = DeviceBuffer(4 * T * n), DeviceBuffer(hip.lib().rl_hip_act_x_bytes(n, T))
+    used = 388 * (n // 128) * T
+    call("rl_hip_rmsnorm_pack", d[0].ptr, n, d[1].ptr, y.ptr, None, n, T, 1e-6, None)
+    call("rl_hip_rmsnorm_x", d[0].ptr, d[1].ptr, x.ptr, n, T, 1e-6, None)
+    call("rl_hip_device_synchronize")
+    want = pack(y.numpy(np.float32, (T, n)))
+    assert x.numpy(np.uint8, (x.nbytes,))[:used].tobytes() == want.numpy(np.uint8, (x.nbytes,))[:used].tobytes()
+    if n < 256:
+        return  # (one head: the norm over all of n)
+    Z = (r.standard_normal((T, n)) * 12).astype(np.float32)
+    z = DeviceBuffer.from_numpy(Z)
+    call("rl_hip_gated_rmsnorm_pack", d[0].ptr, z.ptr, n, d[1].ptr, 128, y.ptr, None, n, T, 1e-6, None)
+    call("rl_hip_gated_rmsnorm_x", d[0].ptr, z.ptr, n, d[1].ptr, x.ptr, n, T, 1e-6, None)
+    call("rl_hip_device_synchronize")
+    want = pack(y.numpy(np.float32, (T, n)))
+    assert x.numpy(np.uint8, (x.nbytes,))[:used].tobytes() == want.numpy(np.uint8, (x.nbytes,))[:used].tobytes()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("fp16,epi,m,n,T", CASES)
 def test_gemm_x(gpu, fp16, epi, m, n, T):
     r = synth.rng(17 * m + n + T + epi)
