@@ -17,7 +17,7 @@
 // gemm_prefill_kernel for BF16 and fp16 tiles (16x16 MFMA).
 #include <type_traits>
 
-#include "internal.h"
+#include "prefill.h"
 
 using namespace rl;
 
@@ -25,12 +25,10 @@ namespace {
 
 constexpr int kPfNT = 2;     // 16-token column tiles per wave
 constexpr int kPfTok = 64 * kPfNT;  // tokens per workgroup
-constexpr int kTileRows = 16;
 
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 union Frag8 {
     bf16x8 v;
@@ -46,29 +44,9 @@ __device__ inline void e4m3x4_to_bf16(uint32_t w, uint32_t& lo, uint32_t& hi) {
     hi = __builtin_bit_cast(uint32_t, b);
 }
 
-__device__ inline float silu_f(float x) { return x / (1.f + __expf(-x)); }
-
 // A barrier that waits for this wave's LDS accesses only (loads to registers stay in
 // flight across it).
 __device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-// Four consecutive outputs (of which `left` exist): one 16-byte access where the row
-// stride and base allow (vec), else one by one.
-__device__ inline void store_rows4(float* dst, const float (&o)[4], int left, int vec, bool add) {
-    if (vec && left >= 4) {
-        float4 r = make_float4(o[0], o[1], o[2], o[3]);
-        float4* d = reinterpret_cast<float4*>(dst);
-        if (add) {
-            const float4 a = *d;
-            r = make_float4(a.x + r.x, a.y + r.y, a.z + r.z, a.w + r.w);
-        }
-        *d = r;
-        return;
-    }
-#pragma unroll
-    for (int v = 0; v < 4; ++v)
-        if (v < left) dst[v] = add ? dst[v] + o[v] : o[v];
-}
 
 // EPI: 0 store, 1 add (Y += W.x), 2 SwiGLU over interleaved gate/up row tiles
 // (even tile = gate rows, odd = up rows of the same 16 outputs; Y row = output row),
@@ -249,7 +227,7 @@ __global__ __launch_bounds__(256) void gemm_prefill_kernel(const uint8_t* __rest
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
                     const float up = __shfl_xor(tot[nt][r][v], 32, 64);
-                    if (g < 2 && orow + v < m_valid) yrow[orow + v] = silu_f(tot[nt][r][v]) * up;
+                    if (g < 2 && orow + v < m_valid) yrow[orow + v] = silu_fast(tot[nt][r][v]) * up;
                 }
             }
         } else if constexpr (EPI == 6) {
@@ -264,7 +242,7 @@ __global__ __launch_bounds__(256) void gemm_prefill_kernel(const uint8_t* __rest
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
                     const float up = __shfl_xor(tot[nt][r][v], 32, 64);
-                    h8[v] = silu_f(tot[nt][r][v]) * up;
+                    h8[v] = silu_fast(tot[nt][r][v]) * up;
                 }
 #pragma unroll
                 for (int v = 0; v < 4; ++v) h8[4 + v] = __shfl_xor(h8[v], 16, 64);
@@ -277,7 +255,7 @@ __global__ __launch_bounds__(256) void gemm_prefill_kernel(const uint8_t* __rest
                 const int orow = ((rt0 + r) / 2) * kTileRows + 4 * g;
 #pragma unroll
                 for (int v = 0; v < 4; ++v)
-                    if (orow + v < m_valid) yrow[orow + v] = silu_f(tot[nt][r][v]) * tot[nt][r + 1][v];
+                    if (orow + v < m_valid) yrow[orow + v] = silu_fast(tot[nt][r][v]) * tot[nt][r + 1][v];
             }
         } else {
 #pragma unroll
@@ -318,15 +296,8 @@ __global__ __launch_bounds__(64 * TG * KW, 2) void gemm_fp8_pf_kernel(const uint
                                                                      int vec) {
     constexpr int kQ = (RT + TG - 1) / TG;  // tiles a wave stages
     constexpr int R2 = RT / 2;
-    // workgroup -> (row block, token block): each XCD (blockIdx % 8) takes a contiguous
-    // run of the order "8 token blocks wide, then down the rows", so the workgroups it
-    // runs at one time share both weights and activations in its L2
-    const int per = gridDim.x / 8;
-    const int lin = (blockIdx.x % 8) * per + blockIdx.x / 8;
-    if (lin >= nrb * ntb) return;
-    const int grp = lin / (nrb * 8), rem = lin - grp * nrb * 8;
-    const int gw = min(8, ntb - grp * 8);
-    const int rb = rem / gw, tb = grp * 8 + rem % gw;
+    int rb, tb;
+    if (!xcd_block(nrb, ntb, 8, rb, tb)) return;
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -524,7 +495,7 @@ __global__ __launch_bounds__(64 * TG * KW, 2) void gemm_fp8_pf_kernel(const uint
                 if (rt + j >= m_tiles) break;
                 float o4[4];
 #pragma unroll
-                for (int v = 0; v < 4; ++v) o4[v] = silu_f(tot[r][8 * j + v]) * tot[r][8 * j + 4 + v];
+                for (int v = 0; v < 4; ++v) o4[v] = silu_fast(tot[r][8 * j + v]) * tot[r][8 * j + 4 + v];
                 if (epi == kEpiSwiGLUHFrag) {
                     // one 8-column fragment unit of the next GEMM's input per tile: lanes h = 0
                     // write its hi part, lanes h = 1 its mid part (the split of pack_act)
@@ -553,7 +524,7 @@ __global__ __launch_bounds__(64 * TG * KW, 2) void gemm_fp8_pf_kernel(const uint
             for (int u = 0; u < 2; ++u) {
                 float o4[4];
 #pragma unroll
-                for (int v = 0; v < 4; ++v) o4[v] = silu_f(tot[r][4 * u + v]) * tot[r][8 + 4 * u + v];
+                for (int v = 0; v < 4; ++v) o4[v] = silu_fast(tot[r][4 * u + v]) * tot[r][8 + 4 * u + v];
                 const int row = (rt / 2) * kTileRows + 8 * u + 4 * h;
                 if (in) store_rows4(yrow + row, o4, m_valid - row, vec, false);
             }

@@ -18,27 +18,22 @@
 // of x, so the 4 bits left of w add 2^-16 of the product).
 #include <type_traits>
 
-#include "internal.h"
+#include "prefill.h"
 
 using namespace rl;
 
 namespace {
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef int i32x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef short s16x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) void lds_void;
-
-constexpr int kTileRows = 16;
 
 union H8u {
     f16x8 v;
     uint32_t u[4];
     i32x4 i;
 };
-
-__device__ inline float silu_f(float x) { return x / (1.f + __expf(-x)); }
 
 // ------------------------------------------------------------- writing inputs
 
@@ -182,24 +177,6 @@ __global__ __launch_bounds__(256) void gnorm_x_kernel(const float* __restrict__ 
 __device__ inline void full_barrier() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 
-// Four consecutive outputs (of which `left` exist): one 16-byte access where the row
-// stride and base allow (vec), else one by one.
-__device__ inline void store_rows4(float* dst, const float (&o)[4], int left, int vec, bool add) {
-    if (vec && left >= 4) {
-        float4 r = make_float4(o[0], o[1], o[2], o[3]);
-        float4* d = reinterpret_cast<float4*>(dst);
-        if (add) {
-            const float4 a = *d;
-            r = make_float4(a.x + r.x, a.y + r.y, a.z + r.z, a.w + r.w);
-        }
-        *d = r;
-        return;
-    }
-#pragma unroll
-    for (int v = 0; v < 4; ++v)
-        if (v < left) dst[v] = add ? dst[v] + o[v] : o[v];
-}
-
 struct GemmX {
     const uint8_t* W;
     const float* ts;
@@ -234,15 +211,8 @@ __global__ __launch_bounds__(128 * TG, 2) void gemm_x_kernel(GemmX p) {
     __shared__ i32x4 A0[RT * kAC * 64], A1[RT * kAC * 64];  // [tile][chunk][lane of the packed tile]
     __shared__ i32x4 B0[NW * 6 * 64], B1[NW * 6 * 64];      // [32 tokens][4 fp16 steps, 2 e4m3 parts][lane]
 
-    // workgroup -> (row block, token block): each XCD (blockIdx % 8) takes a contiguous run
-    // of the order "GW token blocks wide, then down the rows", so the workgroups it runs at
-    // one time share both weights and activations in its L2
-    const int per = gridDim.x / 8;
-    const int lin = (blockIdx.x % 8) * per + blockIdx.x / 8;
-    if (lin >= p.nrb * p.ntb) return;
-    const int grp = lin / (p.nrb * GW), rem = lin - grp * p.nrb * GW;
-    const int gw = min(GW, p.ntb - grp * GW);
-    const int rb = rem / gw, tb = grp * GW + rem % gw;
+    int rb, tb;
+    if (!xcd_block(p.nrb, p.ntb, GW, rb, tb)) return;
 
     const int T = p.T, n_kb = p.n_kb;
     const int lane = threadIdx.x & 63;
@@ -450,7 +420,7 @@ __global__ __launch_bounds__(128 * TG, 2) void gemm_x_kernel(GemmX p) {
 #pragma unroll
                 for (int j = 0; j < 2; ++j)
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) tot[r][n][8 * j + v] = silu_f(tot[r][n][8 * j + v]) * tot[r][n][8 * j + 4 + v];
+                    for (int v = 0; v < 4; ++v) tot[r][n][8 * j + v] = silu_fast(tot[r][n][8 * j + v]) * tot[r][n][8 * j + 4 + v];
         if constexpr (R == 4) {
             if (p.epi == kEpiSwiGLUHX) {
                 // the workgroup's 128 outputs are one column block of the next input: its
