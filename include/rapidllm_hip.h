@@ -110,7 +110,9 @@ int rl_hip_pack_act(const float* X, void* frag, int n, int T, void* stream);
  * buffer.  Deterministic: partial sums are combined in a fixed order, and token t's
  * result does not depend on T. */
 /* Prompt prefill: Y[t][ldy] (=, +=) W . x_t for T (any) tokens of rl_hip_pack_act
- * fragments, on the matrix cores (128 rows x 64 tokens per workgroup).  epilogue:
+ * fragments, on the matrix cores.  Deterministic, but the order of a row's sums (and so
+ * its last bits) depends on T, m and n: with few tokens or rows the waves of a workgroup
+ * split n.  epilogue:
  * 0 store, 1 add, 2 SwiGLU over interleaved gate/up 16-row tiles (m/2 output rows),
  * 5 SwiGLU over the rl_hip_pack_fp8_gate_up half tiles (m/2 output rows), 6 the same
  * written as rl_hip_pack_act fragments of the m/2 outputs (Y is then the fragment

@@ -141,7 +141,8 @@ typedef __attribute__((address_space(3))) void lds_void;
 // leave the wave's registers.  The scores of the next 64 positions are computed while the
 // current ones go through exp.  One wave per SIMD: q fragments and output take 256
 // registers.
-// Bound by that wave's chain: 3072 MFMA cycles in about 5000 per 64 positions.  With 16
+// Bound by that wave's chain: 3072 MFMA cycles in about 7000 per 64 positions (2.15 GHz; 1500
+// tokens over 4000 positions: the matrix cores are busy 36% of the launch).  With 16
 // tokens x 3 heads per workgroup on 16x16 MFMA, K and V from the L2 and P through LDS, 1500
 // tokens over 4000 positions took 514 us (24 / 4 heads), 4092 over 32092 11.3 ms; now 244
 // us and 4.5 ms.  A running maximum that moves only past 2^8 saves the rescaling but

@@ -232,7 +232,13 @@ class Engine {
     const void* pf_f16_src_ = nullptr;
     size_t pf_attn_ws_bytes_ = 0;
     int* pf_pos_ = nullptr;
-    // inputs as fp16 + e4m3 parts (prefill_x.hip), for chunks of at least kPfXMin tokens
+    // Inputs as fp16 + e4m3 parts (prefill_x.hip), for chunks of at least kPfXMin tokens.  Four
+    // layers of the 27B model, chunk of T tokens, ms with these inputs (with bf16 hi + mid):
+    // Q4_K T 17 5.04 (5.30), 63 5.07 (5.68), 64 5.09 (5.72), 256 5.52 (6.85), 796 9.04 (13.6);
+    // block-FP8 17 3.20 (1.88), 63 3.27 (2.25), 64 3.28 (2.28), 128 3.40 (3.02), 256 3.79 (3.37),
+    // 396 4.49 (4.44), 512 4.69 (4.72), 796 5.93 (6.43).  K-quant gains at every size.  Block-FP8,
+    // whose other kernel splits K over idle waves, gains time from about 500 tokens on; between
+    // 64 and there it has these inputs for half the rounding error, at up to 1.4 times the time.
     static constexpr int kPfXMin = 64;
     void *pf_fx_ = nullptr, *pf_fxh_ = nullptr;
     bool pf_use_x_ = false;  // the current chunk's linears take them

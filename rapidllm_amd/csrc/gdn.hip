@@ -134,7 +134,7 @@ __global__ __launch_bounds__(256) void gdn_decode_kernel(GdnArgs p) {
     }
 
     // ---- conv1d over T tokens for the 2*128 q/k channels of the source k-head and
-    // the 32 v channels of this workgroup (288 channels, 256 threads).
+    // the 16 v channels of this workgroup (272 channels, 256 threads).
     // The q/k window state is written back only by one workgroup per source head.
     const bool owns_qk = cg == 0 && (p.v_tiled ? (h == src) : (h == src * rep));
     for (int ch = tid; ch < 2 * kDK + kCols; ch += 256) {

@@ -3,9 +3,8 @@
 // Same arithmetic as ops::gemv_fp8 (reference src/kernels/ops.cpp:182-194) applied
 // to every prompt token, i.e. the reference's prefill linears
 // (src/kernels/cuda/cuda_engine.cu:18338-18590 launch_prefill_chunk -> launch_linear
-// for T > 8, cuda_engine.cu:12008-12016).  At prefill sizes the work is
-// matrix-core bound, not HBM bound: one 128-row x 128-token output block per
-// workgroup reads each weight tile once for 128 tokens.
+// for T > 8, cuda_engine.cu:12008-12016).  At prefill sizes the work is matrix-core
+// bound, not HBM bound; at few tokens it is the weight stream, and waves split K.
 //
 // Operands: A = weight rows, e4m3 decoded to bf16 by the hardware converter (exact); B =
 // tokens of the activation fragments (bf16 hi and mid parts, two MFMAs into the same
@@ -52,9 +51,8 @@ __device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_b
 // (even tile = gate rows, odd = up rows of the same 16 outputs; Y row = output row),
 // 5 SwiGLU over half tiles (tile k: gate rows 8k..8k+7, up rows 8k..8k+7; scales
 // [tile][kb][2]).
-// WK: the weight tiles.  1: BF16 (4 KiB
-// tiles of the decode GEMM's BF16 layout, no scales).  2: two BF16 matrices W_hi +
-// W_lo (a weight split into 16 significant bits): three MFMAs per step,
+// WK: the weight tiles.  1: BF16 (4 KiB tiles of the decode GEMM's BF16 layout, no
+// scales).  2: two BF16 matrices W_hi + W_lo (a weight split into 16 significant bits): three MFMAs per step,
 // hi.x_hi + hi.x_mid + lo.x_hi.  3: fp16 tiles in the BF16 layout with one
 // power-of-two scale per (tile, column block) (the K-quant linears as dequantised
 // for prefill), activations as fp16 hi + lo fragments with one power-of-two scale

@@ -4,14 +4,21 @@
 // here.  A matrix-core product with 16 significant bits of x needs two passes over the
 // weights' operands; with x = hi + mid in bf16 (prefill.hip) both run at the 16-bit
 // rate.  fp16 holds 11 of the bits, so the remainder fits e4m3's 4 and its pass runs at
-// the 8-bit rate: 3/4 of the matrix-core time, 3/4 of the activation bytes, and half
-// the error (rms 4.9e-6 against 9.8e-6 of x: both parts are rounded, not truncated).
+// the 8-bit rate: 3/4 of the matrix-core time and 3/4 of the activation bytes.  Error of a
+// product apart from the weights' rounding (normal inputs, channels 12 to 1e6 times as
+// large, SwiGLU outputs, log-normal ones up to sigma 2): block-FP8 4.9e-6 (bf16 hi + mid, which
+// truncates: 9.8e-6), fp16 tiles, whose second pass rounds the weights, too, 7.3e-6 (two fp16
+// passes over the same truncated x: 9.8e-6).
 //
 // An input of T tokens and n columns (ActX, act_x_bytes):
 //   s [kb][T]        power of two per (128-column block, token) that puts the block's
 //                    largest |x| / s in [2^12, 2^13)
 //   h [kb][i][g][T]  16-byte units, fp16(x / s) of columns 32g + 8i .. + 7
 //   l [kb][c][g][T]  16-byte units, e4m3((x / s - h) * 2^7) of columns 32g + 16c .. + 15
+// One s serves a block, so elements 2^-14 and more below their block's largest lose bits of
+// l (absolute error 2^-29 of the largest), and from 2^-18 on hold the 11 bits of h; bf16 hi +
+// mid keep 16 bits of each.  Only an output that the block's large elements do not reach
+// (weights of 0) can show it.
 // Weights: block-FP8 tiles, decoded to fp16 w * 2^7 for the first pass and taken as they
 // are for the second; or the fp16 tiles of rl_hip_kquant_to_f16, taken as they are for
 // the first and converted to e4m3(w / 2^7) for the second (the remainder carries 2^-12
@@ -195,8 +202,8 @@ struct GemmX {
 // multiply each half block's fp32 partial.
 // WK 0: block-FP8 tiles; 3: fp16 tiles.  kGuh (WK 0): two scales per tile.
 //
-// Bound by matrix-core power and issue: the MFMA units are 60% busy while a round runs,
-// at 1.9 GHz; without any copy into LDS after the first block (timing only) a launch is
+// Bound by matrix-core power and issue: 34816 x 5120, 2044 tokens, block-FP8: MFMA units 60%
+// busy at 1.8 GHz, 7.6 VALU instructions per MFMA, no LDS conflicts; without any copy into LDS after the first block (timing only) a launch is
 // 14% shorter, with every copy hitting the same cache lines 7%.  34816 x 5120, 2044
 // tokens, SwiGLU to inputs: block-FP8 1071 us (680 TFLOP/s of useful products; 1200 us
 // for the bf16 hi + mid kernel), fp16 tiles 1049 us (2300 us for two fp16 passes on
