@@ -124,6 +124,13 @@ int rl_hip_gemm_x(int fp16_tiles, const void* w, const float* tile_scale, const 
                   int T, int epilogue, int ldy, void* stream);
 int rl_hip_gemm_x_split(int fp16_tiles, int epilogue, int m, int T, int cus, int* split);
 
+/* rl_hip_attn_prefill_layer as the engine calls it: *pos_dev + T is known to be at most
+ * max_keys, and the host chooses the kernels (0: the device, from *pos_dev). */
+int rl_hip_attn_prefill_layer_keys(const float* Y, int ld_y, const float* q_norm, const float* k_norm, uint16_t* k_cache,
+                                   uint16_t* vt_cache, int ctx, const int* pos_dev, int T, int n_q, int n_kv, int head_dim,
+                                   int rotary_dim, float theta, float eps, void* workspace, size_t workspace_bytes,
+                                   float* out, int max_keys, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -475,9 +475,17 @@ int rl_hip_attn_prefill_layer(const float* Y, int ld_y, const float* q_norm, con
                               uint16_t* vt_cache, int ctx, const int* pos_dev, int T, int n_q, int n_kv, int head_dim,
                               int rotary_dim, float theta, float eps, void* workspace, size_t workspace_bytes,
                               float* out, void* stream) {
+    return rl_hip_attn_prefill_layer_keys(Y, ld_y, q_norm, k_norm, k_cache, vt_cache, ctx, pos_dev, T, n_q, n_kv, head_dim,
+                                          rotary_dim, theta, eps, workspace, workspace_bytes, out, 0, stream);
+}
+
+int rl_hip_attn_prefill_layer_keys(const float* Y, int ld_y, const float* q_norm, const float* k_norm, uint16_t* k_cache,
+                                   uint16_t* vt_cache, int ctx, const int* pos_dev, int T, int n_q, int n_kv, int head_dim,
+                                   int rotary_dim, float theta, float eps, void* workspace, size_t workspace_bytes,
+                                   float* out, int max_keys, void* stream) {
     return guard([&] {
         rl::attn_prefill_layer(Y, ld_y, q_norm, k_norm, k_cache, vt_cache, ctx, pos_dev, T, n_q, n_kv, head_dim,
-                               rotary_dim, theta, eps, workspace, workspace_bytes, out, S(stream));
+                               rotary_dim, theta, eps, workspace, workspace_bytes, out, S(stream), max_keys);
     });
 }
 

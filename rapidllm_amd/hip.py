@@ -144,6 +144,8 @@ _SIGS = {
     "rl_hip_gated_rmsnorm_x": (_i, [_vp, _vp, _i, _vp, _vp, _i, _i, C.c_float, _vp]),
     "rl_hip_gemm_x": (_i, [_i, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp]),
     "rl_hip_gemm_x_split": (_i, [_i, _i, _i, _i, _i, C.POINTER(_i)]),
+    "rl_hip_attn_prefill_layer_keys": (_i, [_vp, _i, _vp, _vp, _vp, _vp, _i, _vp, _i, _i, _i, _i, _i, C.c_float,
+                                            C.c_float, _vp, _sz, _vp, _i, _vp]),
     "rl_hip_time_gemm_kquant": (_i, [_i, _vp, _i, _vp, _vp, _vp, _sz, _i, _i, _i, _i, _vp, C.POINTER(C.c_float)]),
     "rl_hip_time_gdn": (_i, [_vp, _i, _vp, _vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i,
                              _i, _vp, C.POINTER(C.c_float)]),

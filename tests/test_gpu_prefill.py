@@ -3,7 +3,8 @@ oracle: block-FP8 linears on the matrix cores, 1e-3 relative L2 per token."""
 import numpy as np
 import pytest
 
-from rapidllm_amd import ops, synth
+from rapidllm_amd import hip, ops, synth
+from rapidllm_amd.hip import DeviceBuffer, call
 
 pytestmark = pytest.mark.gpu
 
@@ -597,3 +598,45 @@ def test_attn_prefill_short_context_in_large_cache(gpu, T, pos, nq, nkv):
     else:
         for t in range(T):
             assert rel_l2(outs[1][t], outs[0][t]) < 1e-3, (t, rel_l2(outs[1][t], outs[0][t]))
+
+
+@pytest.mark.parametrize("T,pos,nq,nkv", [
+    (1, 5000, 24, 4), (17, 3001, 24, 4), (33, 1100, 6, 1), (64, 4031, 24, 4), (100, 2503, 12, 2), (65, 1800, 8, 8),
+    (31, 900, 9, 3), (130, 640, 24, 4), (767, 9, 24, 4), (1380, 700, 24, 4)])
+@pytest.mark.parametrize("known", [True, False])
+@pytest.mark.parametrize("whole_ws", [True, False])
+def test_attn_prefill_known_keys_and_small_workspace(gpu, T, pos, nq, nkv, known, whole_ws):
+    """The routes of a chunk past 768 keys: the keys known to the host (as in the engine: the
+    norm / RoPE pass and the merge of their own) or read on the device, in a workspace of the
+    documented size or of the q fragments alone (no split), against single tokens' decode
+    attention over the caches that the chunk left.  The decode kernel and the prefill
+    kernels each round probabilities to fp16 (2^-12) and norm a token's own q in another order:
+    5e-4 each, 1e-3 together.  Nothing is written past the workspace or the output, and a
+    second call gives the same bytes."""
+    r = synth.rng(130 + pos + T + nq)
+    hd, ld, guard = 256, 2 * nq * 256 + 2 * nkv * 256, 4096
+    ctx = 8192
+    Y = r.standard_normal((T, ld)).astype(np.float32)
+    K = r.standard_normal((pos, nkv, hd)).astype(np.float16).astype(np.float32)
+    V = r.standard_normal((pos, nkv, hd)).astype(np.float16).astype(np.float32)
+    qn, kn = (r.standard_normal(hd).astype(np.float32) * np.float32(0.1) for _ in range(2))
+    cache = ops.AttnCache(nkv, ctx, hd)
+    cache.fill(K, V)
+    nb = hip.lib().rl_hip_attn_prefill_workspace_bytes(nq, T) if whole_ws else nq * -(-T // 16) * 16384 + 256
+    ws = DeviceBuffer.from_numpy(np.full(nb + guard, 0xA5, np.uint8))
+    ob = 4 * T * nq * hd
+    out = DeviceBuffer.from_numpy(np.full(ob + guard, 0xA5, np.uint8))
+    args = [DeviceBuffer.from_numpy(a) for a in (Y, qn, kn, np.array([pos], np.int32))]
+    got = []
+    for _ in range(2):
+        call("rl_hip_attn_prefill_layer_keys", args[0].ptr, ld, args[1].ptr, args[2].ptr, cache.k.ptr, cache.vt.ptr, ctx,
+             args[3].ptr, T, nq, nkv, hd, 64, 1e7, 1e-6, ws.ptr, nb, out.ptr, pos + T if known else 0, None)
+        raw = out.numpy(np.uint8, (ob + guard,))
+        assert (raw[ob:] == 0xA5).all() and (ws.numpy(np.uint8, (nb + guard,))[nb:] == 0xA5).all()
+        got.append(raw[:ob].tobytes())
+    assert got[0] == got[1]
+    o = np.frombuffer(got[0], np.float32).reshape(T, nq * hd)
+    assert np.isfinite(o).all()
+    for t in sorted({0, T // 2, T - 1} | {x for x in (15, 16, 31, 32, 63, 64, 1279, 1280) if x < T}):
+        want = ops.attn_decode_layer(Y[t], cache, pos + t, qn, kn, nq, nkv)[0]
+        assert rel_l2(o[t], want) < 1e-3, (t, rel_l2(o[t], want))
