@@ -6,9 +6,9 @@
 // rate.  fp16 holds 11 of the bits, so the remainder fits e4m3's 4 and its pass runs at
 // the 8-bit rate: 3/4 of the matrix-core time and 3/4 of the activation bytes.  Error of a
 // product apart from the weights' rounding (normal inputs, channels 12 to 1e6 times as
-// large, SwiGLU outputs, log-normal ones up to sigma 2): block-FP8 4.9e-6 (bf16 hi + mid, which
-// truncates: 9.8e-6), fp16 tiles, whose second pass rounds the weights, too, 7.3e-6 (two fp16
-// passes over the same truncated x: 9.8e-6).
+// large, log-normal ones of sigma 1 to 6): block-FP8 4.7e-6 to 5.1e-6 (bf16 hi + mid, which
+// truncates: 8.6e-6 to 1.03e-5), fp16 tiles, whose second pass rounds the weights, too,
+// 7.1e-6 to 7.9e-6 (two fp16 passes over the same truncated x: as bf16 hi + mid).
 //
 // An input of T tokens and n columns (ActX, act_x_bytes):
 //   s [kb][T]        power of two per (128-column block, token) that puts the block's
