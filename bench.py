@@ -771,6 +771,10 @@ def main():
     t0 = time.perf_counter()
     eng.prefill(ids)
     pf_s = time.perf_counter() - t0
+    # Steady clocks for the T=4 window too: straight after the one prompt it reads 6.9-7.05 ms,
+    # a second of work later 6.7 (the timed prompt alone gave that while it took longer).
+    for _ in range(4):
+        eng.prefill(ids)
     # T=4 MTP verify (drafts in the token buffer; acceptance advances 1..4)
     eng.synthetic_context(CTX)
     eng.time_steps(4, W)
