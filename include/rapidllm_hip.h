@@ -285,10 +285,9 @@ int rl_hip_embed_rows(const void* table, int kind, const int* tokens_dev, float*
  * follows *pos_dev at each replay).  The workspace holds the q fragments and 34 MB for
  * the split; one of only n_q * ceil(T/16) * 16 KiB + 256 bytes is accepted and nothing is
  * split.  Outputs are the same from call to call, but the order of a token's sums
- * depends on T and on the number of keys.  Masked positions have probability 0, not no
- * part: an infinity or NaN in a token's V (also one past fp16's range) can reach the tokens
- * before it in the same call that share its workgroup and stage: at most 94, with
- * n_q = n_kv 158.  Replaces the reference's prefill attention
+ * depends on T and on the number of keys.  An infinity or NaN in a token's V (also one past
+ * fp16's range) reaches that token and later ones; up to 768 keys, where a masked position takes
+ * part with probability 0, also up to 46 tokens before it.  Replaces the reference's prefill attention
  * (cuda_engine.cu:18338-18590; CPU: per token ops::attn_decode, ops.cpp:575-605). */
 size_t rl_hip_attn_prefill_workspace_bytes(int n_q, int T);
 int rl_hip_attn_prefill_layer(const float* Y, int ld_y, const float* q_norm, const float* k_norm, uint16_t* k_cache,

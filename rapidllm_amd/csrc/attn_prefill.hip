@@ -6,6 +6,7 @@
 // cache with a running max / sum / output per query (online softmax), and
 // attn_merge_kernel adds the parts of the queries whose positions were split.
 #include <algorithm>
+#include <climits>
 
 #include "attn.h"
 
@@ -153,6 +154,7 @@ __global__ __launch_bounds__(256, 1) void attn_prefill_kernel(AttnArgs p, const 
     if (auto_route && attn_prefill_auto_short(*p.pos + p.T)) return;  // attn_prefill_finish_kernel has it
     __shared__ i32x4 K0[2048], K1[2048];  // [d/32][pos/16][(d/8)%4][pos%16]
     __shared__ i32x4 V0[2048], V1[2048];  // [pos/32][d/16][(pos/8)%4][d%16]
+    __shared__ int flag[4];
     // kv head from the XCD (blockIdx % 8), so that its cache is read through one L2 (or
     // two); longest items first
     int kv, idx;
@@ -181,6 +183,7 @@ __global__ __launch_bounds__(256, 1) void attn_prefill_kernel(AttnArgs p, const 
     const int qpos = p0 + min(tok, p.T - 1);
     const int L = pf_keys(items - 1 - idx, p.G, p.T, p0);  // keys 0 .. L-1 for the workgroup
     const int q_first = p0 + 32 * tb;                       // positions up to here need no mask
+    const int wg_first = p0 + 32 * ((items - 1 - idx) * 4 / p.G);  // ... in any wave
     const int nblk = (L + 63) / 64;
     const int parts = split ? pf_parts(pp.parts, nblk) : 1;
     if (part >= parts) return;
@@ -237,9 +240,7 @@ __global__ __launch_bounds__(256, 1) void attn_prefill_kernel(AttnArgs p, const 
     f32x16 o[8], s[2], z;
 #pragma unroll
     for (int v = 0; v < 16; ++v) z[v] = 0.f;
-#pragma unroll
-    for (int dt = 0; dt < 8; ++dt) o[dt] = z;
-    float m = -INFINITY, l = 0.f;  // running max of the scaled scores (log2 units), lane's part of the sum
+    float m, l;  // running max of the scaled scores (log2 units), lane's part of the sum
 
     // K row 8u + 4h' + v of a 32-position tile is position 16 (u / 2) + 8 h' + 4 (u % 2) + v
     const int krow = 8 * ((col >> 2) & 1) + 4 * ((col >> 3) & 1) + (col & 3);
@@ -274,9 +275,7 @@ __global__ __launch_bounds__(256, 1) void attn_prefill_kernel(AttnArgs p, const 
         return fmaxf(x, __shfl_xor(x, 32, 64)) * c;
     };
     auto step = [&](int blk, float mx, const i32x4* Kn, const i32x4* V) {
-        // (the first block moves m from -inf: o and l are 0; a lane whose positions are all
-        // masked in this part keeps a finite m, probabilities of 0 and a sum of 0)
-        const float mn = fmaxf(fmaxf(m, mx), -1e30f);
+        const float mn = fmaxf(m, mx);
         const float alpha = __builtin_amdgcn_exp2f(m - mn);
         l *= alpha;
         m = mn;
@@ -319,23 +318,89 @@ __global__ __launch_bounds__(256, 1) void attn_prefill_kernel(AttnArgs p, const 
         return mask_max(blk + 1, s);
     };
 
-    dma_k(blk0, K0);
-    dma_k(blk0 + 1, K1);
-    dma_v(blk0, V0);
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    scores(K0, s);
-    float mx = mask_max(blk0, s);
-    // block blk: K(blk + 1) and V(blk) are in LDS; K(blk + 2) and V(blk + 1) on their way
-    for (int blk = blk0; blk < blk1; blk += 2) {
+    // The non-finite V of a block that some query masks: to the outputs of the queries that see
+    // their position, and zeros for the product.
+    auto clean_v = [&](int blk, i32x4* V) {
+        const uint16_t* vh = reinterpret_cast<const uint16_t*>(V);
+#pragma unroll 1
+        for (int j = 0; j < 64; ++j) {
+            const uint16_t* row = vh + (j >> 5) * 8192 + ((j >> 3) & 3) * 128 + (j & 7);
+            const uint32_t see = 64 * blk + j <= qpos ? 0xffffu : 0u;
+            bool bad = false;
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                bad |= (row[(lane >> 2) * 512 + (4 * (lane & 3) + k) * 8] & 0x7c00u) == 0x7c00u;
+            if (__ballot(bad) == 0) continue;
+#pragma unroll
+            for (int dt = 0; dt < 8; ++dt)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    const int d = 32 * dt + 8 * (v >> 2) + (v & 3);
+                    const uint32_t x = row[(d >> 4) * 512 + ((d & 15) + 4 * h) * 8] & see;
+                    const float add = static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(x)));
+                    o[dt][v] += (x & 0x7c00u) == 0x7c00u ? add : 0.f;
+                }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll 1
+        for (int q = 0; q < 8; ++q) {
+            i32x4 x = V[wave * 512 + q * 64 + lane];
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+                const uint32_t w = static_cast<uint32_t>(x[d]);
+                const uint32_t m16 = ((((w & 0x7c007c00u) + 0x04000400u) >> 15) & 0x00010001u) * 0xffffu;
+                x[d] = static_cast<int>(w & ~m16);
+            }
+            V[wave * 512 + q * 64 + lane] = x;
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    };
+
+    // A masked probability is 0, and 0 times an infinity or NaN a NaN: non-finite V of later tokens
+    // (or left in the cache behind them) would reach queries that do not see it.  A workgroup
+    // with an output that is not finite starts again and takes such values out of the blocks
+    // with masks.  That costs the others the check of their outputs and a looser schedule of
+    // the loop: 2% (1000 tokens over 9000 positions 426 -> 435 us).  Measured instead: every
+    // workgroup scanning its blocks with masks 3 us a call or 7%, a loop of its own for the
+    // second pass 4%, a function call for it 13 us (scratch memory).
+    int clean_from = INT_MAX;  // the position from which blocks are cleaned: the second pass's
+    for (;;) {
+        l = 0.f;
+#pragma unroll
+        for (int dt = 0; dt < 8; ++dt) o[dt] = z;
+        dma_k(blk0, K0);
+        dma_k(blk0 + 1, K1);
+        dma_v(blk0, V0);
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        dma_k(blk + 2, K0);
-        dma_v(blk + 1, V1);
-        mx = step(blk, mx, K1, V0);
-        if (blk + 1 >= blk1) break;
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        dma_k(blk + 3, K1);
-        dma_v(blk + 2, V0);
-        mx = step(blk + 1, mx, K0, V1);
+        scores(K0, s);
+        float mx = mask_max(blk0, s);
+        m = fmaxf(mx, -1e30f);  // (a lane whose positions are all masked in this part: probabilities and a sum of 0)
+        // block blk: K(blk + 1) and V(blk) are in LDS; K(blk + 2) and V(blk + 1) on their way
+        for (int blk = blk0; blk < blk1; blk += 2) {
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            if (__builtin_expect(64 * blk + 63 > clean_from, 0)) clean_v(blk, V0);
+            dma_k(blk + 2, K0);
+            dma_v(blk + 1, V1);
+            mx = step(blk, mx, K1, V0);
+            if (blk + 1 >= blk1) break;
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            if (__builtin_expect(64 * blk + 127 > clean_from, 0)) clean_v(blk + 1, V1);
+            dma_k(blk + 3, K1);
+            dma_v(blk + 2, V0);
+            mx = step(blk + 1, mx, K0, V1);
+        }
+        if (clean_from != INT_MAX) break;
+        float t[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int dt = 0; dt < 8; ++dt)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) t[v & 3] = fmaf(o[dt][v], 0.f, t[v & 3]);
+        const bool any = __ballot((t[0] + t[1]) + (t[2] + t[3]) != 0.f) != 0;
+        if (lane == 0) flag[wave] = any;
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (__builtin_amdgcn_readfirstlane(flag[0] | flag[1] | flag[2] | flag[3]) == 0) break;
+        asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+        clean_from = wg_first;
     }
 
     l += __shfl_xor(l, 32, 64);

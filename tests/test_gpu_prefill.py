@@ -640,3 +640,41 @@ def test_attn_prefill_known_keys_and_small_workspace(gpu, T, pos, nq, nkv, known
     for t in sorted({0, T // 2, T - 1} | {x for x in (15, 16, 31, 32, 63, 64, 1279, 1280) if x < T}):
         want = ops.attn_decode_layer(Y[t], cache, pos + t, qn, kn, nq, nkv)[0]
         assert rel_l2(o[t], want) < 1e-3, (t, rel_l2(o[t], want))
+
+
+@pytest.mark.parametrize("T,pos,nq,nkv,bad", [
+    (200, 1000, 24, 4, (100, 199)), (900, 1000, 24, 4, (0, 97, 640)), (130, 800, 6, 1, (31, 32)),
+    (300, 700, 8, 8, (140, 299)), (70, 4003, 9, 3, (47,)), (1400, 33, 24, 4, (64, 1024, 1399)), (1, 900, 24, 4, (0,))])
+@pytest.mark.parametrize("known", [True, False])
+def test_attn_prefill_non_finite_v(gpu, T, pos, nq, nkv, bad, known):
+    """Infinities and NaN in the V of some tokens (some dims of one kv head), past 768 keys:
+    they reach that token's outputs and those after it, in these dims, and leave every other
+    output byte as it is without them."""
+    r = synth.rng(170 + pos + T + nq)
+    hd, ctx = 256, 8192
+    Y = r.standard_normal((T, 2 * nq * hd + 2 * nkv * hd)).astype(np.float32)
+    K, V = (r.standard_normal((pos, nkv, hd)).astype(np.float16).astype(np.float32) for _ in range(2))
+    qn, kn = (r.standard_normal(hd).astype(np.float32) * np.float32(0.1) for _ in range(2))
+    kv = nkv - 1
+    v0 = 2 * nq * hd + nkv * hd + kv * hd
+    Yb = Y.copy()
+    Yb[bad[0], v0 + 3] = np.inf
+    Yb[bad[0], v0 + 129] = -np.inf
+    Yb[bad[-1], v0 + 3] = np.inf
+    Yb[bad[-1], v0 + 250] = np.nan
+    Yb[bad[-1], v0 + 64] = -1e5  # past fp16's range
+    outs = []
+    for y in (Y, Yb):
+        cache = ops.AttnCache(nkv, ctx, hd)
+        cache.fill(K, V)
+        ws = DeviceBuffer(hip.lib().rl_hip_attn_prefill_workspace_bytes(nq, T))
+        out = DeviceBuffer(4 * T * nq * hd)
+        args = [DeviceBuffer.from_numpy(a) for a in (y, qn, kn, np.array([pos], np.int32))]
+        call("rl_hip_attn_prefill_layer_keys", args[0].ptr, y.shape[1], args[1].ptr, args[2].ptr, cache.k.ptr, cache.vt.ptr,
+             ctx, args[3].ptr, T, nq, nkv, hd, 64, 1e7, 1e-6, ws.ptr, ws.nbytes, out.ptr, pos + T if known else 0, None)
+        outs.append(out.numpy(np.float32, (T, nkv, nq // nkv, hd)))
+    want = outs[0]
+    for t, d, x in ((bad[0], 3, np.inf), (bad[0], 129, -np.inf), (bad[-1], 250, np.nan), (bad[-1], 64, -np.inf)):
+        want[t:, kv, :, d] = x
+    assert np.array_equal(want.view(np.uint32)[~np.isnan(want)], outs[1].view(np.uint32)[~np.isnan(want)])
+    assert np.isnan(outs[1][np.isnan(want)]).all()
